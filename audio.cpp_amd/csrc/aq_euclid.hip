@@ -11,6 +11,7 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <utility>
 #include <vector>
 
 namespace {
@@ -176,6 +177,19 @@ __global__ void euclid_prep_kernel(const float *__restrict__ cbf, int64_t QN, in
     if (nf) nonfinite[0] = 1;
 }
 
+// The fp16 codebook in the matrix cores' fragment order: [N/16][K/32][64]
+// pieces of 8, lane l's piece of (block, slice) holding row 16 block + l % 16,
+// elements 32 slice + 8 (l / 16).  A wave's fragment is 1 KB in a row: read
+// from the row-major image, its lanes hit 64 different 16-byte pieces and a
+// CU took 72 K cycles for a 1 MB codebook (14 bytes a cycle).
+__global__ void euclid_fragments_kernel(const u32x4 *__restrict__ cbh, int64_t pieces, int K, u32x4 *__restrict__ cbx) {
+    const int64_t o = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (o >= pieces) return;
+    const int ks = K / 32, l = static_cast<int>(o % kWave);
+    const int64_t row = o / kWave / ks * 16 + l % 16;
+    cbx[o] = cbh[row * (K / 8) + o / kWave % ks * 4 + l / 16];
+}
+
 // --------------------------------------------------------------- dispatch
 
 const KsKernels *kernels_for(int ks) {
@@ -212,6 +226,7 @@ struct aq_codebooks {
     bool any = false;
     uint16_t *d_cbh = nullptr;   // [Q][N][K] fp16(c)
     uint16_t *d_cbl = nullptr;   // [Q][N][K] fp16(c - fp16(c)) (refine pass)
+    uint16_t *d_cbx = nullptr;   // d_cbh in fragment order (K = 256: the narrow cascade)
     float *d_hh = nullptr;       // [Q][N] -|c|^2 / 2 (fp32 of the double sum)
     float *d_cbf = nullptr;      // [Q][N][K]
     float *d_bias = nullptr;     // [Q][N] (OMNI)
@@ -258,7 +273,8 @@ aq_status check_upload(aq_ctx *ctx, const char *fn, int64_t Q, int64_t N, int64_
 }
 
 // A codebook set with its device buffers allocated, not yet filled.
-aq_status euclid_alloc(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, bool q8, int recipe, aq_codebooks **out) {
+aq_status euclid_alloc(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, bool q8, bool any, int recipe,
+                       aq_codebooks **out) {
     aq_codebooks *cb = new (std::nothrow) aq_codebooks();
     if (!cb) return aq_fail(ctx, AQ_E_NOMEM, "aq_euclid_upload: host allocation failed");
     cb->device = ctx->device;
@@ -267,10 +283,12 @@ aq_status euclid_alloc(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, bool q8, in
     cb->K = K;
     cb->recipe = recipe;
     cb->q8 = q8;
+    cb->any = any;
     const size_t QNK = static_cast<size_t>(Q * N * K), QN = static_cast<size_t>(Q * N);
     bool ok = hipMalloc(&cb->d_cbh, QNK * 2) == hipSuccess && hipMalloc(&cb->d_cbl, QNK * 2) == hipSuccess &&
               hipMalloc(&cb->d_hh, QN * 4) == hipSuccess && hipMalloc(&cb->d_cbf, QNK * 4) == hipSuccess &&
               hipMalloc(&cb->d_bias, QN * 4) == hipSuccess && hipMalloc(&cb->d_e2, QN * 4) == hipSuccess;
+    if (ok && !any && K == 256) ok = hipMalloc(&cb->d_cbx, QNK * 2) == hipSuccess;
     if (ok && q8) ok = hipMalloc(&cb->d_q8, QNK) == hipSuccess && hipMalloc(&cb->d_q8d, QNK / 32 * 4) == hipSuccess;
     if (!ok) {
         aq_euclid_release(cb);
@@ -339,6 +357,12 @@ aq_status euclid_prepare(aq_ctx *ctx, aq_codebooks *cb) {
         hipLaunchKernelGGL(euclid_prep_kernel, grid, block, 0, ctx->stream, cb->d_cbf, QN, cb->N,
                            static_cast<int>(cb->K), cb->d_cbh, cb->d_cbl, cb->d_hh, cb->d_bias, cb->d_e2, smax,
                            nonfinite);
+        if (cb->d_cbx) {
+            const int64_t pieces = QN * cb->K / 8;
+            hipLaunchKernelGGL(euclid_fragments_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
+                               ctx->stream, reinterpret_cast<const u32x4 *>(cb->d_cbh), pieces,
+                               static_cast<int>(cb->K), reinterpret_cast<u32x4 *>(cb->d_cbx));
+        }
         step = "launch";
         e = hipGetLastError();
         if (e == hipSuccess) {
@@ -398,8 +422,7 @@ aq_status euclid_upload_from(aq_ctx *ctx, const char *fn, int64_t Q, int64_t N, 
     if (st != AQ_OK) return st;
     aq_device_guard g(ctx->device);
     aq_codebooks *cb = nullptr;
-    st = euclid_alloc(ctx, Q, N, K, cb_type != AQ_CB_F32, recipe, &cb);
-    if (st == AQ_OK) cb->any = any;
+    st = euclid_alloc(ctx, Q, N, K, cb_type != AQ_CB_F32, any, recipe, &cb);
     if (st == AQ_OK) st = euclid_fill(ctx, cb, cb_type, data, kind);
     if (st == AQ_OK) st = euclid_prepare(ctx, cb);
     if (st != AQ_OK) {
@@ -449,9 +472,8 @@ aq_status aq_euclid_upload_ema(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, con
     aq_device_guard g(ctx->device);
     const size_t QNK = static_cast<size_t>(Q * N * K), QN = static_cast<size_t>(Q * N);
     aq_codebooks *cb = nullptr;
-    st = euclid_alloc(ctx, Q, N, K, false, recipe, &cb);
+    st = euclid_alloc(ctx, Q, N, K, false, any, recipe, &cb);
     if (st != AQ_OK) return st;
-    cb->any = any;
     // the inputs go to the device once; the codebook is materialised straight
     // into the set's fp32 buffer and prepared there
     float *d = nullptr;
@@ -517,7 +539,7 @@ aq_status aq_euclid_release(aq_codebooks *cb) {
         aq_device_guard g(cb->device);
         aq_proj_release(cb->proj);
         for (void *p : {static_cast<void *>(cb->d_cbh), static_cast<void *>(cb->d_cbl), static_cast<void *>(cb->d_hh),
-                        static_cast<void *>(cb->d_cbf),
+                        static_cast<void *>(cb->d_cbx), static_cast<void *>(cb->d_cbf),
                         static_cast<void *>(cb->d_bias), static_cast<void *>(cb->d_e2), static_cast<void *>(cb->d_q8),
                         static_cast<void *>(cb->d_q8d), static_cast<void *>(cb->d_bounds)})
             if (p) (void)hipFree(p);
@@ -668,24 +690,41 @@ aq_status euclid_encode_any(aq_ctx *ctx, const aq_codebooks *cb, const aq_frames
     return AQ_OK;
 }
 
-// The encode pipeline of a plain codebook: the register-resident one-launch
-// cascade where it exists (K = 256), else the per-stage pipeline.  The
-// one-launch cascade that keeps the residual in memory measured no faster
-// than the per-stage pipeline at K = 256 and slower for Q8_0 codebooks (its
+// The encode pipeline of a plain codebook: the narrow one-launch cascade
+// where it exists (K = 256), else the per-stage pipeline.  The one-launch
+// cascade that keeps the residual in memory measured no faster than the
+// per-stage pipeline at K = 256 and slower for Q8_0 codebooks (its
 // verification then scans 2-3 % of the frames); it runs when
 // AQ_EUCLID_PIPELINE=cascade asks for it (comparisons and tests), as
-// AQ_EUCLID_PIPELINE=stages asks for the per-stage pipeline.
-enum class Pipeline { kStages, kCascade, kResident };
-Pipeline pipeline_for(const aq_codebooks *cb, const KsKernels *kk, int var, int topl) {
+// AQ_EUCLID_PIPELINE=stages asks for the per-stage pipeline and narrow1,
+// narrow2, narrow4 for the narrow cascade at that many frame groups.
+//
+// Frame groups per block: a round of blocks (one per CU) takes about 110, 120
+// and 157 us with one, two and four groups (8 stages of 2048 codes; the same
+// proportions for Q8_0 and DIRECT), so the count with the least rounds x time
+// runs: up to 16 frames per CU one group, up to 32 two, else mostly four.
+enum class Pipeline { kStages, kCascade, kNarrow };
+Pipeline pipeline_for(const aq_codebooks *cb, const KsKernels *kk, int var, int topl, int64_t M, int cus, int *fg) {
     if (cb->proj || cb->exact_only || !kk->cascade[var][topl - 3]) return Pipeline::kStages;
     const char *e = std::getenv("AQ_EUCLID_PIPELINE");
     if (e && std::strcmp(e, "stages") == 0) return Pipeline::kStages;
     if (e && std::strcmp(e, "cascade") == 0) return Pipeline::kCascade;
-    return kk->resident[var][topl - 3] ? Pipeline::kResident : Pipeline::kStages;
+    if (!cb->d_cbx) return Pipeline::kStages;
+    int64_t best = INT64_MAX;
+    for (const auto &[groups, cost] : {std::pair<int, int>{1, 110}, {2, 120}, {4, 157}}) {
+        const int64_t frames = int64_t{16} * groups * cus;
+        const int64_t c = (M + frames - 1) / frames * cost;
+        if (c <= best) {
+            best = c;
+            *fg = groups;
+        }
+    }
+    if (e && std::strncmp(e, "narrow", 6) == 0 && std::strchr("124", e[6]) && e[6]) *fg = e[6] - '0';
+    return Pipeline::kNarrow;
 }
 
 // Encode with a one-launch cascade: every stage of every frame in
-// euclid_resident_kernel (resident) or euclid_cascade_kernel (frames the
+// euclid_narrow_kernel or euclid_cascade_kernel (frames the
 // certificate cannot settle continue with their best exact candidate and
 // are listed), the exact verification of the listed (frame, stage) pairs
 // (their values spread over the grid, then the selections), and the fix-up
@@ -694,17 +733,18 @@ Pipeline pipeline_for(const aq_codebooks *cb, const KsKernels *kk, int var, int 
 aq_status euclid_encode_cascade(aq_ctx *ctx, const aq_codebooks *cb, const aq_frames_desc &in, int64_t M, int32_t *idx,
                                 float *residual, float *dist, int topk, int32_t *topk_idx, float *topk_dist,
                                 const int32_t *force_idx, Arena &arena, const KsKernels *kk, int var, int topl,
-                                bool resident) {
+                                Pipeline pipe, int fg) {
     const int K = static_cast<int>(cb->K);
     CascadeFn casc = kk->cascade[var][topl - 3], ver = kk->verify[var], fix = kk->fixup[var];
     CascadeFn vvals = kk->verify_values[var];
     size_t clds = static_cast<size_t>(kk->cascade_lds);
     int frames = kk->cascade_frames, threads = kCThreads;
-    if (resident) {
-        casc = kk->resident[var][topl - 3];
-        clds = static_cast<size_t>(kk->resident_lds);
-        frames = kk->resident_frames;
-        threads = kRsThreads;
+    if (pipe == Pipeline::kNarrow) {
+        const NarrowKernels *nk = kernels_narrow(fg);
+        casc = nk->fn[var][topl - 3];
+        clds = static_cast<size_t>(nk->lds[var][topl - 3]);
+        frames = nk->frames;
+        threads = kNwThreads;
     }
     const size_t slds = scan_lds_bytes(K);
     {
@@ -798,6 +838,7 @@ aq_status euclid_encode_cascade(aq_ctx *ctx, const aq_codebooks *cb, const aq_fr
     }
     c.x0 = x0;
     c.work = work;
+    c.cbx = cb->d_cbx;
     c.bounds = cb->d_bounds;
     c.counts = ints;
     c.bad_count = ints + 129;
@@ -855,10 +896,11 @@ aq_status euclid_encode_impl(aq_ctx *ctx, const aq_codebooks *cb, const aq_frame
     const int topl = topk >= 4 ? 4 : 3;
     const KsKernels *kk = kernels_for(ks);
     const int var = variant_of(cb->recipe, cb->q8);
-    const Pipeline pipe = pipeline_for(cb, kk, var, topl);
+    int fg = 0;
+    const Pipeline pipe = pipeline_for(cb, kk, var, topl, M, ctx->num_cus > 0 ? ctx->num_cus : 256, &fg);
     if (pipe != Pipeline::kStages)
         return euclid_encode_cascade(ctx, cb, in, M, idx, residual, dist, topk, topk_idx, topk_dist, force_idx, arena, kk,
-                                     var, topl, pipe == Pipeline::kResident);
+                                     var, topl, pipe, fg);
     StageFn sweep = kk->sweep[cb->q8 ? 1 : 0][topl - 3];
     StageFn select = kk->select[var][topl - 3];
     StageFn scan = kk->exact_scan[var];

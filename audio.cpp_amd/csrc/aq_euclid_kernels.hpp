@@ -235,6 +235,7 @@ struct CascadeArgs {
     int32_t *bad_count;      // frames listed in bad_list
     int32_t *bad_list;       // [M]
     int write_last;          // the last stage writes the residual
+    const uint16_t *cbx;     // [Q][N/16][K/32][64][8] fp16 codebook in fragment order (narrow cascade)
 };
 
 using StageFn = void (*)(StageArgs);
@@ -276,12 +277,15 @@ struct KsKernels {
     CascadeFn fixup[4];
     int cascade_lds;          // cascade dynamic LDS bytes (TOPL 4)
     int cascade_frames;       // frames per cascade block
-    // The register-resident cascade (the widths whose residual fits the
-    // registers; null otherwise).
-    CascadeFn resident[4][2]; // [variant][topl]
-    int resident_lds;         // its dynamic LDS bytes (TOPL 4)
-    int resident_frames;      // frames per block
 };
+// The narrow cascade at K = 256 (aq_euclid_narrow.hip): [variant][topl], its
+// dynamic LDS and frames per block, for FG = 1, 2, 4 frame groups.
+struct NarrowKernels {
+    CascadeFn fn[4][2];
+    int lds[4][2];
+    int frames;
+};
+const NarrowKernels *kernels_narrow(int fg);
 const KsKernels *kernels_ks2();
 const KsKernels *kernels_ks8();
 const KsKernels *kernels_ks16();
@@ -716,6 +720,73 @@ __device__ inline float row_ror_add(float v) {
     return __fadd_rn(v, __int_as_float(o));
 }
 
+// One (frame, code) pair per quad of lanes, lane q holding elements
+// 16 l + 4 q + t of every 16-element step (16-byte reads, 64 bytes in a row
+// per quad).  quad_step adds a step to acc, quad_value gives the whole sum
+// in every lane of the quad.
+//  * tinyBLAS order: acc[t] is accumulator 4 q + t; then
+//    _mm512_reduce_add_ps's pairing tree: lanes q, q ^ 2 hold accumulators
+//    j, j + 8, then lanes 0, 1 t3[j], t3[j + 4].
+//  * DIRECT: the rounded squares are added in element order, the running sum
+//    (acc[0]) handed from lane to lane by quad permutations, so that a pair
+//    costs 24 VALU instructions per 16 elements and a wave reads 16 rows
+//    coalesced (a pair per lane: 48, and 64 rows scattered).
+template <int RECIPE>
+__device__ inline void quad_step(f32x4 &acc, const f32x4 &c, const f32x4 &x) {
+    if constexpr (RECIPE == DIRECT) {
+        float s[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float d = __fsub_rn(x[t], c[t]);
+            s[t] = __fmul_rn(d, d);
+        }
+        float d = acc[0];
+#define AQ_QUAD_TURN(CTRL)                                                                                       \
+        d = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(d), CTRL, 0xF, 0xF, false));            \
+        d = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(d, s[0]), s[1]), s[2]), s[3]);
+        AQ_QUAD_TURN(0xFF)   // lane 0 takes lane 3's sum of the step before
+        AQ_QUAD_TURN(0x00)
+        AQ_QUAD_TURN(0x55)
+        AQ_QUAD_TURN(0xAA)
+#undef AQ_QUAD_TURN
+        acc[0] = d;
+    } else {
+        constexpr float sa = RECIPE == OMNI ? 2.0f : 1.0f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t] = __fmaf_rn(c[t] * sa, x[t], acc[t]);
+    }
+}
+template <int RECIPE>
+__device__ inline float quad_value(const f32x4 &acc) {
+    if constexpr (RECIPE == DIRECT) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[0]), 0xFF, 0xF, 0xF, false));
+    } else {
+        float t6[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float v = __fadd_rn(acc[t], __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc[t]), 0x4E, 0xF, 0xF, false)));
+            t6[t] = __fadd_rn(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false)));
+        }
+        return __fadd_rn(__fadd_rn(t6[0], t6[2]), __fadd_rn(t6[1], t6[3]));
+    }
+}
+// The per-code term of the recipe (OmniVoice's bias, Higgs's |c|^2) and the
+// recipe's value from the pair's sum, that term and the frame's
+// sum_rows(x*x).
+template <int RECIPE>
+__device__ inline float quad_term(const StageArgs &a, int n) {
+    return RECIPE == OMNI ? a.bias[n] : (RECIPE == HIGGS ? a.e2[n] : 0.0f);
+}
+template <int RECIPE>
+__device__ inline float quad_recipe(float v, float term, float x2) {
+    if (RECIPE == OMNI) return __fadd_rn(v, term);
+    if (RECIPE == HIGGS) return __fsub_rn(__fsub_rn(__fmul_rn(v, 2.0f), x2), term);
+    return v;
+}
+// Whether a stage's exact values take the quad form.
+template <int RECIPE, bool Q8>
+__device__ inline bool quad_form(const StageArgs &a) { return !Q8 && (RECIPE == DIRECT || a.order == 0); }
+
 // ggml's hsum_float_8 ((a0+a4) + (a2+a6)) + ((a1+a5) + (a3+a7)) of eight
 // accumulators held by 8 neighbouring lanes, lane j holding a_{q8_lane_word(j)}
 // (words 0, 1, 2, 3, 7, 6, 5, 4): the half-row mirror pairs a_i with a_{i+4},
@@ -778,13 +849,31 @@ __device__ inline float rows_sum(float x) {
 // quantize_row_q8_0: d = fp16(amax/127), q = round-half-even(x * 127/amax)),
 // held by 4 lanes 16 apart with 8 elements each.  x_q is exact in fp32
 // (a 7-bit integer times an fp16 scale).
-__device__ inline void q8_image_block(float (&v)[8]) {
+// The lane's 8 quants go to xq and the scale to xd where given.
+__device__ inline void q8_image_block(float (&v)[8], int8_t *xq = nullptr, float *xd = nullptr) {
     float am = 0.0f;
 #pragma unroll
     for (int t = 0; t < 8; ++t) am = fmaxf(am, fabsf(v[t]));
     am = rows_max(am);
-    const float dq = static_cast<float>(static_cast<_Float16>(__fdiv_rn(am, 127.0f)));
-    const float id = am != 0.0f ? __fdiv_rn(127.0f, am) : 0.0f;
+    float dq, id;
+    q8_scale(am, dq, id);
+    if (xq) {
+        int q[8];
+        if (am < INFINITY && id < INFINITY) {
+            // |v * id| <= 127 (1 + 2^-23)^2: the rounded values are integers
+            // in [-127, 127], where q8_quant's range test and clamp are idle
+            // (a frame holding a NaN is not certified and reads none of this)
+#pragma unroll
+            for (int t = 0; t < 8; ++t) q[t] = static_cast<int>(__builtin_rintf(__fmul_rn(v[t], id)));
+        } else {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) q[t] = q8_quant(v[t], id);
+        }
+        int *w = reinterpret_cast<int *>(xq);
+        w[0] = q8_pack4(q[0], q[1], q[2], q[3]);
+        w[1] = q8_pack4(q[4], q[5], q[6], q[7]);
+        *xd = dq;
+    }
 #pragma unroll
     for (int t = 0; t < 8; ++t) v[t] = __fmul_rn(__builtin_rintf(__fmul_rn(v[t], id)), dq);
 }
@@ -1068,14 +1157,23 @@ __global__ __launch_bounds__(kThreads, sweep_blocks_per_cu(KS)) void euclid_swee
 // exactly, the frames' sum_rows(x*x) and (Q8_0) their query blocks, XQS
 // bytes apart: the 8 lane groups of a pass read 8 frames' blocks, which a
 // stride of K + 32 bytes puts in different LDS banks.
-template <bool Q8, int K, int TOPL>
+// With PRE the block holds the frames' sums and query blocks elsewhere.
+template <bool Q8, int K, int TOPL, bool PRE = false>
 struct SelLds {
     static constexpr int QCAP = 16 * 4 * TOPL;
     static constexpr int XQS = K + 32;
-    alignas(16) int8_t q_xq[Q8 ? 16 * XQS : 16];
-    float q_xd[Q8 ? 16 * (K / 32) : 1];
+    alignas(16) int8_t q_xq[Q8 && !PRE ? 16 * XQS : 16];
+    float q_xd[Q8 && !PRE ? 16 * (K / 32) : 1];
     int32_t q_n[QCAP], q_f[QCAP];
-    float q_v[QCAP], q_x2[16];
+    float q_v[QCAP], q_x2[PRE ? 1 : 16];
+};
+// The terms of a group's frames that PRE passes to select_group: their
+// sum_rows(x*x) (Higgs) and Q8_0 query blocks (rows SelLds::XQS apart) and
+// scales.
+struct SelPre {
+    const float *x2;
+    const int8_t *xq;
+    const float *xd;
 };
 
 // Certificate, exact re-ranking, outputs and residual update of one group of
@@ -1089,11 +1187,13 @@ struct SelLds {
 // a.spec_list as (frame, stage) for the exact verification after the
 // cascade.  With `update` the residual a.xout = a.xin - c[code] is written
 // for the settled frames; the lane's frame's code is returned (-1: frame
-// not settled or past M).
-template <int RECIPE, bool Q8, int KS, int TOPL>
+// not settled or past M).  Only the frames of `fmask` (bit f: frame f) are
+// settled, so that several waves can share a group's frames.
+template <int RECIPE, bool Q8, int KS, int TOPL, bool PRE = false>
 __device__ int select_group(const StageArgs &a, int64_t m_base, const float (&top_in)[TOPL], float taul_in,
-                            float nx2_in, float nd2_in, float nxx2_in, SelLds<Q8, KS * 32, TOPL> &sl,
-                            bool speculate, const float *xrows, int xstride, bool update) {
+                            float nx2_in, float nd2_in, float nxx2_in, SelLds<Q8, KS * 32, TOPL, PRE> &sl,
+                            bool speculate, const float *xrows, int xstride, bool update, unsigned fmask = 0xFFFFu,
+                            SelPre pre = {}) {
     constexpr int K = KS * 32;
     constexpr int FG = 1;
     const int lane = threadIdx.x & (kWave - 1);
@@ -1124,9 +1224,10 @@ __device__ int select_group(const StageArgs &a, int64_t m_base, const float (&to
     int32_t *q_n = sl.q_n;
     int32_t *q_f = sl.q_f;
     float *q_v = sl.q_v;
-    float *q_x2 = sl.q_x2;
-    int8_t *q_xq = sl.q_xq;
-    float *q_xd = sl.q_xd;
+    // written below unless PRE
+    float *q_x2 = PRE ? const_cast<float *>(pre.x2) : sl.q_x2;
+    int8_t *q_xq = PRE ? const_cast<int8_t *>(pre.xq) : sl.q_xq;
+    float *q_xd = PRE ? const_cast<float *>(pre.xd) : sl.q_xd;
 
     float Eg[FG], taug[FG], best0g[FG];
     bool okg[FG], needg[FG];
@@ -1135,7 +1236,7 @@ __device__ int select_group(const StageArgs &a, int64_t m_base, const float (&to
 #pragma unroll
     for (int g = 0; g < FG; ++g) {
         const int64_t m = m_base + g * 16 + col;
-        const bool live = m < a.M;
+        const bool live = m < a.M && ((fmask >> col) & 1u) != 0;
 
         // Bound E (in units of v = x.c - |c|^2/2) on |v(n) - S'(n)| for every n.
         const float nx = sqrtf(nx2[g]) * 1.0001f, nd = sqrtf(nd2[g]) * 1.0001f;
@@ -1149,39 +1250,43 @@ __device__ int select_group(const StageArgs &a, int64_t m_base, const float (&to
         const float trunc = ldexpf(vmax, lbits - 23);
         const float E = 1.02f * (e_half + e_acc + e_rec + 4.0f * u * vmax) + trunc + 1e-30f;
 
-        // Keys of the frame's 4 lanes, gathered in every one of them.
-        float all[4 * TOPL];
-#pragma unroll
-        for (int j = 0; j < TOPL; ++j) {
-            float kr[4];
-            rows4(top[g][j], kr);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) all[4 * j + q] = kr[q];
-        }
         // tau bounds every key a lane dropped; vT is the T-th largest kept key.
-        float tau = taul[g];
-        tau = rows_max(tau);
-        float best[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+        const float tau = rows_max(taul[g]);
+        float vT, best0;
+        if (Tk == 1) {
+            vT = best0 = rows_max(top[g][0]);
+        } else {
+            // keys of the frame's 4 lanes, gathered in every one of them
+            float best[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
-        for (int t = 0; t < 4 * TOPL; ++t) {
-            float v = all[t];
+            for (int j = 0; j < TOPL; ++j) {
+                float kr[4];
+                rows4(top[g][j], kr);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float hi = fmaxf(best[r], v);
-                v = fminf(best[r], v);
-                best[r] = hi;
+                for (int q = 0; q < 4; ++q) {
+                    float v = kr[q];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float hi = fmaxf(best[r], v);
+                        v = fminf(best[r], v);
+                        best[r] = hi;
+                    }
+                }
             }
+            vT = best[Tk - 1];
+            best0 = best[0];
         }
-        const float vT = best[Tk - 1];
         const bool ok = live && !a.exact_only && (E < INFINITY) && (vT - vT == 0.0f);
         const float thr = vT - 2.0f * E;
-        int nabove = 0;
+        int above[4], nabove = 0;   // the frame's keys at or above the threshold
 #pragma unroll
-        for (int t = 0; t < 4 * TOPL; ++t) nabove += all[t] >= thr ? 1 : 0;
+        for (int j = 0; j < TOPL; ++j) nabove += top[g][j] >= thr ? 1 : 0;
+        rows4(nabove, above);
+        nabove = (above[0] + above[1]) + (above[2] + above[3]);
         const bool need = ok && (want_value || nabove > 1);
         Eg[g] = E;
         taug[g] = tau;
-        best0g[g] = best[0];
+        best0g[g] = best0;
         okg[g] = ok;
         needg[g] = need;
         // enqueue this lane's candidates
@@ -1210,7 +1315,8 @@ __device__ int select_group(const StageArgs &a, int64_t m_base, const float (&to
     // elements (lane kq the 64 from 64 kq), add their squares in order in
     // turn (the double running sum handed on from lane to lane) and quantise
     // their two blocks from registers.
-    if (RECIPE == HIGGS && K % 256 == 0) {
+    if (PRE) {
+    } else if (RECIPE == HIGGS && K % 256 == 0) {
         if (__any(needg[0])) {
             static_assert(FG == 1, "one frame group per select wave");
             const int fq = m_base + col < a.M ? col : static_cast<int>(a.M - 1 - m_base);
@@ -1296,47 +1402,32 @@ __device__ int select_group(const StageArgs &a, int64_t m_base, const float (&to
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     // 2c: exact values of the queued pairs, in the reference's arithmetic.
-    if (!Q8 && RECIPE != DIRECT && a.order == 0) {
-        // tinyBLAS: 16 accumulators over k = 16 l + j, one per lane of a
-        // 16-lane row (coalesced row reads), then _mm512_reduce_add_ps's
-        // pairing tree as DPP row rotations 8, 4, 2, 1; 4 pairs per pass.
-        // Several pairs per row and pass (four up to K = 256, else two), so
-        // that their row reads are in flight together.
-        constexpr int P = K <= 256 ? 4 : 2;
-        const int j = lane & 15, grp = lane >> 4;
-        const float sa = RECIPE == OMNI ? 2.0f : 1.0f;
-        for (int e0 = grp; e0 < qcount; e0 += 4 * P) {
-            int fs[P], n[P];
-            float acc[P], off[P];
+    if (quad_form<RECIPE, Q8>(a)) {
+        // a pair per quad, 16 pairs a pass; the row reads of 256 elements are
+        // issued together
+        constexpr int LB = K / 16 < 16 ? K / 16 : 16;   // 16-element steps
+        static_assert(K / 16 % LB == 0, "whole batches");
+        const int q = lane & 3;
+        for (int e0 = 0; e0 < qcount; e0 += 16) {
+            const int e = e0 + lane / 4;
+            const int fs = e < qcount ? q_f[e] : 0;
+            const int n = e < qcount ? q_n[e] : 0;
+            const float term = quad_term<RECIPE>(a, n);   // loaded with the row, not after the sum
+            const float *cr = a.cbf + static_cast<int64_t>(n) * K + 4 * q;
+            const float *xr = xrows + static_cast<int64_t>(fs) * xstride + 4 * q;
+            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int p = 0; p < P; ++p) {
-                const int e = e0 + 4 * p;
-                fs[p] = e < qcount ? q_f[e] : 0;
-                n[p] = e < qcount ? q_n[e] : 0;
-                acc[p] = 0.0f;
+            for (int l0 = 0; l0 < K / 16; l0 += LB) {
+                f32x4 cv[LB];
+#pragma unroll
+                for (int l = 0; l < LB; ++l) cv[l] = *reinterpret_cast<const f32x4 *>(cr + 16 * (l0 + l));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int l = 0; l < LB; ++l)
+                    quad_step<RECIPE>(acc, cv[l], *reinterpret_cast<const f32x4 *>(xr + 16 * (l0 + l)));
             }
-            // the code's bias (OmniVoice) or |c|^2 (Higgs) is loaded with
-            // its row, not after the sum
-#pragma unroll
-            for (int p = 0; p < P; ++p) off[p] = RECIPE == OMNI ? a.bias[n[p]] : a.e2[n[p]];
-#pragma unroll
-            for (int l = 0; l < K / 16; ++l)
-#pragma unroll
-                for (int p = 0; p < P; ++p)
-                    acc[p] = __fmaf_rn(a.cbf[static_cast<int64_t>(n[p]) * K + 16 * l + j] * sa,
-                                       xrows[static_cast<int64_t>(fs[p]) * xstride + 16 * l + j], acc[p]);
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                float v = row_ror_add<8>(acc[p]);
-                v = row_ror_add<4>(v);
-                v = row_ror_add<2>(v);
-                v = row_ror_add<1>(v);
-                const int e = e0 + 4 * p;
-                if (j == 0 && e < qcount) {
-                    if (RECIPE == OMNI) q_v[e] = __fadd_rn(v, off[p]);
-                    else q_v[e] = __fsub_rn(__fsub_rn(__fmul_rn(v, 2.0f), q_x2[fs[p]]), off[p]);
-                }
-            }
+            const float v = quad_value<RECIPE>(acc);
+            if (q == 0 && e < qcount) q_v[e] = quad_recipe<RECIPE>(v, term, RECIPE == HIGGS ? q_x2[fs] : 0.0f);
         }
     } else if (Q8) {
         // ggml_vec_dot_q8_0_q8_0: 8 accumulators over the 4-element groups
@@ -1415,7 +1506,7 @@ __device__ int select_group(const StageArgs &a, int64_t m_base, const float (&to
 #pragma unroll
     for (int g = 0; g < FG; ++g) {
         const int64_t m = m_base + g * 16 + col;
-        const bool live = m < a.M;
+        const bool live = m < a.M && ((fmask >> col) & 1u) != 0;
         bool ok = okg[g];
         const float E = Eg[g], tau = taug[g];
         const float x2 = RECIPE == HIGGS ? q_x2[g * 16 + col] : 0.0f;
@@ -1904,16 +1995,12 @@ __device__ void heap_walk(const float *src, int N, int *hn, float *hv) {
 // ---------------------------------------------------- spread exact values
 // The exact values of every code of up to scap open frames, spread over the
 // grid: item (slot, chunk) writes svals[slot][chunk codes].  F32 codebooks
-// in tinyBLAS order take four lanes per code (lane q of a quad accumulates
-// k = 16 l + 4 q + t, t < 4: tinyBLAS lanes 4q .. 4q+3) and kScanQuadCodes
-// codes per item, every row and frame read issued at once, then reduce16's
-// tree across the quad (lanes q, q ^ 2 hold accumulators j, j + 8; lanes 0,
-// 1 then hold t3[j], t3[j + 4]).  Otherwise a code per thread, kScanThreads
+// in tinyBLAS order and DIRECT take four lanes per code (quad_step) and
+// kScanQuadCodes codes per item, every row and frame read issued at once.
+// Otherwise a code per thread, kScanThreads
 // codes per item, from the frame staged in xs (its Q8_0 blocks in xq, xd)
 // while the block stays on one slot (cur).  x2s: the frame's
 // sum_rows(x*x) (Higgs).  Called by every thread of a kScanThreads block.
-template <int RECIPE, bool Q8>
-__device__ inline bool spread_quad(const StageArgs &a) { return !Q8 && RECIPE != DIRECT && a.order == 0; }
 // Whether the open frames of a stage skip the split pass: at most scap of
 // them, and their exact values read at most kDirectElems codebook elements
 // (count * N * K; 64 MiB of fp32 rows), above which the split pass, which
@@ -1924,7 +2011,7 @@ __device__ inline bool direct_scan(const StageArgs &a, int count, int K) {
 }
 template <int RECIPE, bool Q8>
 __device__ inline int spread_chunks(const StageArgs &a) {
-    const int cpi = spread_quad<RECIPE, Q8>(a) ? kScanQuadCodes : kScanThreads;
+    const int cpi = quad_form<RECIPE, Q8>(a) ? kScanQuadCodes : kScanThreads;
     return (a.N + cpi - 1) / cpi;
 }
 // The quad path's values of one chunk of codes for the frame xr (global
@@ -1937,10 +2024,9 @@ __device__ void quad_values(const StageArgs &a, float *out, int chunk, const flo
         const int q = tid & 3;
         const int nc = n < a.N ? n : a.N - 1;
         const float *cr = a.cbf + static_cast<int64_t>(nc) * K;
-        const float sa = RECIPE == OMNI ? 2.0f : 1.0f;
         // up to 256 elements' reads in flight at once (32 float4 registers)
         constexpr int KC = K < 256 ? K : 256;
-        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int k0 = 0; k0 < K; k0 += KC) {
             f32x4 vc[KC / 16], vx[KC / 16];
@@ -1950,23 +2036,11 @@ __device__ void quad_values(const StageArgs &a, float *out, int chunk, const flo
                 vx[l] = *reinterpret_cast<const f32x4 *>(xr + k0 + 16 * l + 4 * q);
             }
 #pragma unroll
-            for (int l = 0; l < KC / 16; ++l)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) acc[t] = __fmaf_rn(vc[l][t] * sa, vx[l][t], acc[t]);
+            for (int l = 0; l < KC / 16; ++l) quad_step<RECIPE>(acc, vc[l], vx[l]);
         }
-        float t3[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) t3[t] = __fadd_rn(__shfl_xor(acc[t], 2), acc[t]);
-        float t6[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) t6[t] = __fadd_rn(__shfl_xor(t3[t], 1), t3[t]);
-        const float dot = __fadd_rn(__fadd_rn(t6[0], t6[2]), __fadd_rn(t6[1], t6[3]));
+        const float v = quad_value<RECIPE>(acc);
         if (RECIPE == HIGGS) __syncthreads();   // x2s
-        if (q == 0 && n < a.N) {
-            const float v = RECIPE == OMNI ? __fadd_rn(dot, a.bias[n])
-                                           : __fsub_rn(__fsub_rn(__fmul_rn(dot, 2.0f), x2s), a.e2[n]);
-            out[n] = v;
-        }
+        if (q == 0 && n < a.N) out[n] = quad_recipe<RECIPE>(v, quad_term<RECIPE>(a, n), x2s);
     }
 }
 // The values of codes [n0, n1) of the frame xs (LDS) into rv[n] by one
@@ -1977,7 +2051,6 @@ template <int RECIPE, int K>
 __device__ void block_values_quad(const StageArgs &a, const float *xs, float x2, float *rv, int n0, int n1) {
     const int tid = threadIdx.x;
     const int q = tid & 3, cl = tid >> 2;
-    const float sa = RECIPE == OMNI ? 2.0f : 1.0f;
     constexpr int U = 2;
     f32x4 vx[K / 16];
 #pragma unroll
@@ -1993,21 +2066,12 @@ __device__ void block_values_quad(const StageArgs &a, const float *xs, float x2,
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int l = 0; l < K / 16; ++l)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) acc[t] = __fmaf_rn(vc[u][l][t] * sa, vx[l][t], acc[t]);
-            float t3[4], t6[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) t3[t] = __fadd_rn(__shfl_xor(acc[t], 2), acc[t]);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) t6[t] = __fadd_rn(__shfl_xor(t3[t], 1), t3[t]);
-            const float dot = __fadd_rn(__fadd_rn(t6[0], t6[2]), __fadd_rn(t6[1], t6[3]));
+            for (int l = 0; l < K / 16; ++l) quad_step<RECIPE>(acc, vc[u][l], vx[l]);
+            const float v = quad_value<RECIPE>(acc);
             const int n = c0 + u * kScanQuadCodes + cl;
-            if (q == 0 && n < n1)
-                rv[n] = RECIPE == OMNI ? __fadd_rn(dot, a.bias[n])
-                                       : __fsub_rn(__fsub_rn(__fmul_rn(dot, 2.0f), x2), a.e2[n]);
+            if (q == 0 && n < n1) rv[n] = quad_recipe<RECIPE>(v, quad_term<RECIPE>(a, n), x2);
         }
     }
 }
@@ -2064,8 +2128,8 @@ template <int RECIPE, bool Q8, int K>
 __device__ void spread_item(const StageArgs &a, int slot, int chunk, int &cur, float *xs, int8_t *xq, float *xd,
                             float &x2s) {
     const int tid = threadIdx.x;
-    constexpr bool kQuadOk = !Q8 && RECIPE != DIRECT;
-    if (kQuadOk && spread_quad<RECIPE, Q8>(a)) {
+    constexpr bool kQuadOk = !Q8;
+    if (kQuadOk && quad_form<RECIPE, Q8>(a)) {
         const int64_t m = a.fail_list[slot];
         const float *xr = a.xin + m * K;
         __syncthreads();   // the previous item's readers of x2s
@@ -2686,10 +2750,7 @@ __device__ inline float wave_sum(float v) {
 
 // Exact values of one frame's candidates cn[0 .. ncand), in exact_value_kq's
 // arithmetic, with several candidates per pass and coalesced row reads:
-//  * tinyBLAS order: 16 lanes per candidate, lane j accumulating the
-//    elements k = 16 l + j, then _mm512_reduce_add_ps's pairing tree as DPP
-//    row rotations 8, 4, 2, 1; two candidates per 16-lane row and pass, so
-//    that their row reads are in flight together;
+//  * tinyBLAS order and DIRECT: a quad of lanes per candidate (quad_step);
 //  * Q8_0 (ggml_vec_dot_q8_0_q8_0): 8 lanes per candidate, lane j taking the
 //    j-th 4-element group of every block, then hsum_float_8 as lane
 //    exchanges 4, 2, 1;
@@ -2698,35 +2759,34 @@ __device__ inline float wave_sum(float v) {
 template <int RECIPE, bool Q8, int K>
 __device__ void exact_values_frame(const StageArgs &a, const float *__restrict__ x, float x2, const int8_t *xq,
                                    const float *xd, const int *cn, float *cv, int ncand, int lane) {
-    if (!Q8 && RECIPE != DIRECT && a.order == 0) {
-        constexpr int P = 2;
-        const int j = lane & 15, grp = lane >> 4;
-        const float sa = RECIPE == OMNI ? 2.0f : 1.0f;
-        for (int c0 = grp; c0 < ncand; c0 += 4 * P) {
-            int n[P];
-            float acc[P];
+    if (quad_form<RECIPE, Q8>(a)) {
+        constexpr int LB = K / 16 < 16 ? K / 16 : 16;   // 16-element steps read together
+        const int q = lane & 3;
+        // ncand is the same in every lane; in a scalar register the loop
+        // leaves the execution mask alone.  (As a loop through the mask that
+        // keeps the whole frame in registers, ROCm 7.2's compiler put the
+        // restores of registers it had moved to AGPRs behind the loop's exit,
+        // where no lane is active, and the next frame was read through a
+        // wrong pointer; the frame is read again for each batch, too.)
+        const int nc = __builtin_amdgcn_readfirstlane(ncand);
+        for (int c0 = 0; c0 < nc; c0 += 16) {
+            const int c = c0 + lane / 4;
+            const int n = cn[c < nc ? c : c0];
+            const float term = quad_term<RECIPE>(a, n);
+            const float *cr = a.cbf + static_cast<int64_t>(n) * K + 4 * q;
+            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int p = 0; p < P; ++p) {
-                const int c = c0 + 4 * p;
-                n[p] = cn[c < ncand ? c : c0];
-                acc[p] = 0.0f;
+            for (int l0 = 0; l0 < K / 16; l0 += LB) {
+                f32x4 v[LB];
+#pragma unroll
+                for (int l = 0; l < LB; ++l) v[l] = *reinterpret_cast<const f32x4 *>(cr + 16 * (l0 + l));
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int l = 0; l < LB; ++l)
+                    quad_step<RECIPE>(acc, v[l], *reinterpret_cast<const f32x4 *>(x + 16 * (l0 + l) + 4 * q));
             }
-#pragma unroll
-            for (int l = 0; l < K / 16; ++l)
-#pragma unroll
-                for (int p = 0; p < P; ++p)
-                    acc[p] = __fmaf_rn(a.cbf[static_cast<int64_t>(n[p]) * K + 16 * l + j] * sa, x[16 * l + j], acc[p]);
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                float v = row_ror_add<8>(acc[p]);
-                v = row_ror_add<4>(v);
-                v = row_ror_add<2>(v);
-                v = row_ror_add<1>(v);
-                const int c = c0 + 4 * p;
-                if (j == 0 && c < ncand)
-                    cv[c] = RECIPE == OMNI ? __fadd_rn(v, a.bias[n[p]])
-                                           : __fsub_rn(__fsub_rn(__fmul_rn(v, 2.0f), x2), a.e2[n[p]]);
-            }
+            const float v = quad_value<RECIPE>(acc);
+            if (q == 0 && c < nc) cv[c] = quad_recipe<RECIPE>(v, term, x2);
         }
     } else if (Q8) {
         const int j = lane & 7, grp = lane >> 3;
@@ -2818,7 +2878,10 @@ __global__ __launch_bounds__(kWave) void euclid_refine_select_kernel(StageArgs a
         const float e_rec = (K + 16) * u * (nxe * a.cmax + nxe * nxe + a.cmax * a.cmax);
         const float vmax = mag + e_acc;
         const float E = 1.02f * (e_split + e_acc + e_rec + 4.0f * u * vmax) + ldexpf(vmax, 6 - 23) + 1e-30f;
-        ok = ok && (E < INFINITY);
+        // ok and ncand are the same in every lane (a block is one wave, E
+        // comes from butterfly sums): in scalar registers, so that no branch
+        // or loop below works through the execution mask
+        ok = __builtin_amdgcn_readfirstlane(ok && (E < INFINITY) ? 1 : 0) != 0;
 
         // Keys of every slice: tau bounds every code a lane dropped; vT is
         // the T-th largest key (ties by position).
@@ -2879,7 +2942,7 @@ __global__ __launch_bounds__(kWave) void euclid_refine_select_kernel(StageArgs a
                 pp = bp;
             }
             vT = pv;
-            ok = (vT - vT == 0.0f);
+            ok = __builtin_amdgcn_readfirstlane(vT - vT == 0.0f ? 1 : 0) != 0;
         }
         if (ok) {
             const float thr = vT - 2.0f * E;
@@ -3314,72 +3377,101 @@ __global__ __launch_bounds__(kCThreads, 1) void euclid_cascade_kernel(CascadeArg
     }
 }
 
-// ------------------------------------------------------------- resident cascade
-// The residual cascade with the residual held in registers.  A block of
-// kRsWaves waves (one per SIMD, up to 512 registers each) owns kRsWaves x FG
-// x 16 frames through all stages.  Wave w keeps the fp32 residual of its FG
-// frame groups in the MFMA fragment layout (lane (col, kq) of group g holds
-// x[16 g + col][32 ks + 8 kq + t], t < 8) and per stage
-//  1. builds the fp16 fragments and rounding norms from it;
-//  2. sweeps the stage's whole codebook through double-buffered LDS chunks
-//     that the block's waves stage together (no code split between waves,
-//     so no merge of key lists);
-//  3. per group: copies the residual rows into its LDS scratch (read by the
-//     exact re-ranking), runs the select (certificate, exact re-ranking and
-//     outputs; a frame the certificate cannot settle continues with its
-//     best evaluated code and is listed for euclid_verify_kernel) and
-//     subtracts the chosen (or forced) code's row in registers.
-// Only the last stage's residual is written to memory.
-constexpr int kRsWaves = 4;
-constexpr int kRsThreads = kRsWaves * kWave;
+// ------------------------------------------------------------ narrow cascade
 
-// The resident residual lives in accumulation registers (AGPRs): the sweep
-// keeps the architectural registers for its fragments, accumulators and
-// key lists, and the residual is read and written only between sweeps.
-__device__ inline float agpr_put(float x) {
-    float a;
-    asm("v_accvgpr_write_b32 %0, %1" : "=a"(a) : "v"(x));
-    return a;
-}
-__device__ inline float agpr_get(float a) {
-    float x;
-    asm("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(a));
-    return x;
-}
+// The residual cascade with the residual on chip (K = 256).  A block takes
+// FG x 16 frames through all stages and its eight waves split the codes: per
+// stage
+//  1. the fp32 residual rows in LDS become fp16 fragments and rounding norms,
+//     wave w converting K-slices w, w + 8, ...; every wave then holds all
+//     the block's fragments;
+//  2. wave w contracts the 16-code blocks w, w + 8, ..., its A fragments read
+//     straight from the fragment-ordered codebook image in device memory (no
+//     two waves share a fragment, so LDS staging would only add a copy),
+//     nw_ring fragments ahead;
+//  3. the waves' key lists meet in LDS, and each wave runs the select of its
+//     share of the frames (select_group's fmask: the exact values of a
+//     frame's few candidates are memory round trips, which the waves take
+//     side by side) and updates their residual rows.  A frame the
+//     certificate cannot settle continues with its best evaluated code and
+//     is listed for euclid_verify_kernel.
+// Only the last stage's residual is written to memory.
+//
+// What bounds it: with one or two groups the codebook stream into the CU
+// (N K 2 bytes a stage, 42 bytes a cycle: 24 K of 31 K cycles a stage), with
+// four the MFMAs and key updates of two waves per SIMD (25 K of 38 K); then
+// the select's round trips.  Blocks share nothing, so the time is the same
+// for any number of blocks up to one per CU: 8 stages of 2048 codes took
+// 125 us for up to 4 096 frames (FG = 1), 129 us for 8 192 (FG = 2), 174 us
+// for 16 384 (FG = 4) and 471 us for 48 000.  The kernel it replaces (192
+// frames per block, each wave sweeping a whole codebook from LDS for its own
+// 48 frames, residual in AGPRs) took 434-502 us for any of these.
+constexpr int kNwWaves = 8;
+constexpr int kNwThreads = kNwWaves * kWave;
+// A fragments in flight per wave (four frame groups leave room for one 16-code block)
+constexpr int nw_ring(int fg) { return fg < 4 ? 16 : 8; }
+
+// Keys per lane while sweeping, for TOPL after the merge.  A wave's list is
+// one of eight for the same codes and loses a candidate only when an eighth
+// of the lane's codes holds as many: four keep what the merge to six does.
+// (Two for three left 3 % of Mimi's frames open: a list's last key bounds
+// what it dropped, so a close second in the best code's own list is enough.)
+constexpr int nw_keys(int topl) { return topl <= 4 ? topl : 4; }
 
 template <int KS, int FG, int TOPL, bool Q8>
-struct RsLayout {
+struct NwLayout {
     static constexpr int K = KS * 32;
-    static constexpr int BUFB = Tile<KS>::CHUNKB + kRsThreads * 4;   // chunk + one |c|^2/2 slot per thread
-    static constexpr int STAGE16 = Tile<KS>::CHUNKB / 16 / kRsThreads;
-    static constexpr int SWEEP = 2 * BUFB;
-    static constexpr int XSTR = K + 4;   // row stride of the scratch rows (floats; padded against bank conflicts)
-    static constexpr int SELB = (static_cast<int>(sizeof(SelLds<Q8, K, TOPL>)) + 15) / 16 * 16;
-    static constexpr int WSCR = SELB + 16 * XSTR * 4;                 // per wave: select queues + 16 rows
-    static constexpr int BYTES = SWEEP > kRsWaves * WSCR ? SWEEP : kRsWaves * WSCR;
-    static constexpr int FRAMES = kRsWaves * FG * 16;
+    static constexpr int FRAMES = FG * 16;
+    static constexpr int XSTR = K + 4;   // residual row stride (floats)
+    static constexpr int ROWS = FRAMES * XSTR * 4;
+    static constexpr int NRM = KS * FRAMES * 3 * 4;              // partial norms per K-slice
+    static constexpr int XH = FG * KS * kWave * 16;              // fp16 fragments
+    static constexpr int KEYS = kNwWaves * FG * nw_keys(TOPL) * kWave * 4;
+    static constexpr int SELB = (static_cast<int>(sizeof(SelLds<Q8, K, TOPL, true>)) + 15) / 16 * 16;
+    static constexpr int XQS = SelLds<Q8, K, TOPL, true>::XQS;
+    static constexpr int XQ = Q8 ? FRAMES * (XQS + KS * 4) : 0;   // query blocks and scales
+    static constexpr int X2 = FRAMES * 4;                         // sum_rows(x*x)
+    // the select queues take the place of the fragments and keys
+    static constexpr int PHASE = XH + KEYS > kNwWaves * SELB ? XH + KEYS : kNwWaves * SELB;
+    static constexpr int BYTES = ROWS + NRM + X2 + XQ + PHASE;
+    static_assert(BYTES <= static_cast<int>(kAqLdsBytes), "a block's LDS");
 };
 
 template <int RECIPE, bool Q8, int KS, int FG, int TOPL>
-__global__ __launch_bounds__(kRsThreads, 1) void euclid_resident_kernel(CascadeArgs c) {
+__global__ __launch_bounds__(kNwThreads, 1) void euclid_narrow_kernel(CascadeArgs c) {
     using T = Tile<KS>;
-    using LY = RsLayout<KS, FG, TOPL, Q8>;
+    using LY = NwLayout<KS, FG, TOPL, Q8>;
     using MX = Mx;
     constexpr int K = T::K;
-    constexpr int BPC = T::CC / 16;                       // 16-code blocks per chunk
-    static_assert(T::CHUNKB % (16 * kRsThreads) == 0, "a chunk splits evenly over the block");
-    constexpr int PPB = (LY::STAGE16 + BPC - 1) / BPC;    // staged pieces per block
+    constexpr int R = nw_ring(FG);
+    constexpr int TS = nw_keys(TOPL);
+    constexpr int U = R > KS ? R / KS : 1;   // 16-code blocks per unrolled step
+    static_assert((U * KS) % R == 0, "the ring's slots are fixed within a step");
+    constexpr int WPG = kNwWaves / FG;       // select waves per frame group
+    constexpr int FPW = 16 / WPG;            // their frames
+    static_assert(kNwWaves % FG == 0, "whole waves per frame group");
+    constexpr int KV = (K + 4 * kWave - 1) / (4 * kWave);   // float4 per lane per row
+    // the next stage's first fragments are loaded behind the update's rows
+    // where the registers hold both, else ahead of the conversion
+    constexpr bool kEarly = !Q8 && FG < 4;
     extern __shared__ __align__(16) unsigned char lds[];
+    float *xr = reinterpret_cast<float *>(lds);                             // [FRAMES][XSTR]
+    float *nrm = reinterpret_cast<float *>(lds + LY::ROWS);                 // [KS][3][FRAMES]
+    float *x2s = reinterpret_cast<float *>(lds + LY::ROWS + LY::NRM);       // [FRAMES]
+    int8_t *xq = reinterpret_cast<int8_t *>(lds + LY::ROWS + LY::NRM + LY::X2);   // [FRAMES][XQS]
+    float *xd = reinterpret_cast<float *>(xq + LY::FRAMES * LY::XQS);             // [FRAMES][KS]
+    unsigned char *phase = lds + LY::ROWS + LY::NRM + LY::X2 + LY::XQ;
+    u32x4 *xh = reinterpret_cast<u32x4 *>(phase);                           // [FG][KS][64]
+    float *keys = reinterpret_cast<float *>(phase + LY::XH);                // [wave][FG][TS][64]
 
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // uniform: addresses stay scalar
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int col = lane & 15, kq = lane >> 4;
     const int64_t M = c.a.M;
     const int N = c.a.N;
     const int64_t m_tile = static_cast<int64_t>(blockIdx.x) * LY::FRAMES;
     if (m_tile >= M) return;   // block-uniform
-    const int64_t m_wave = m_tile + wave * (FG * 16);
-    for (int i = threadIdx.x; i < LY::FRAMES; i += kRsThreads)
+    for (int i = threadIdx.x; i < LY::FRAMES; i += kNwThreads)
         if (m_tile + i < M) c.bad_stage[m_tile + i] = c.a.Q;
 
     int lbits = 0;   // bits of the lane-local code index (N/4 codes per lane)
@@ -3387,48 +3479,64 @@ __global__ __launch_bounds__(kRsThreads, 1) void euclid_resident_kernel(CascadeA
     const unsigned kmask = (1u << lbits) - 1u;
     unsigned vkeep;
     asm volatile("v_mov_b32 %0, %1" : "=v"(vkeep) : "s"(~kmask));
-    const int nch = N / T::CC;
-    constexpr int R = KS % 4 == 0 ? 4 : 2;
-    constexpr int L = R - 1;
-    constexpr int kWaitLoads = 0x0070;   // s_waitcnt vmcnt(0) lgkmcnt(0)
-    const int hsrc = threadIdx.x < T::CC ? threadIdx.x : 0;
-    const StageOffsets<T, kRsThreads> so;
+    const int nblk = N / 16;
+    const int nb = wave < nblk ? (nblk - wave + kNwWaves - 1) / kNwWaves : 0;   // this wave's 16-code blocks
 
-    // the stage-0 input, in the fragment layout (rows past M read row M - 1),
-    // held in AGPRs
-    float xr[FG][KS][8];
+    // the stage-0 input (rows past M read row M - 1)
+    for (int e = threadIdx.x; e < LY::FRAMES * (K / 4); e += kNwThreads) {
+        const int f = e / (K / 4), k = e % (K / 4) * 4;
+        const int64_t m = m_tile + f < M ? m_tile + f : M - 1;
+        *reinterpret_cast<f32x4 *>(xr + f * LY::XSTR + k) = *reinterpret_cast<const f32x4 *>(c.x0 + m * K + k);
+    }
+
+    typename MX::V8 ring[R];
+    f32x4 hring[U];
+    // block i of this wave (past its last: the last again, whose keys are
+    // not inserted)
+    auto blk_of = [&](int i) { return wave + kNwWaves * (i < nb ? i : nb - 1); };
+    auto load_a = [&](const uint16_t *cbx, int i, int ks) -> typename MX::V8 {
+        return reinterpret_cast<const typename MX::V8 *>(cbx)[(static_cast<int64_t>(blk_of(i)) * KS + ks) * kWave + lane];
+    };
+    auto load_h = [&](const float *nhh, int i) -> f32x4 {
+        return *reinterpret_cast<const f32x4 *>(nhh + blk_of(i) * 16 + kq * 4);
+    };
+    auto fill = [&](const uint16_t *cbx, const float *nhh) {
+        if (nb > 0) {
+            // the loop's order (a block's constants, then its fragments), so
+            // that the waits at its head hold on entry too
 #pragma unroll
-    for (int g = 0; g < FG; ++g) {
-        const int64_t m = m_wave + g * 16 + col;
-        const float *row = c.x0 + (m < M ? m : M - 1) * K;
+            for (int u = 0; u < U; ++u) {
+                hring[u] = load_h(nhh, u);
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const f32x4 lo = *reinterpret_cast<const f32x4 *>(row + ks * 32 + kq * 8);
-            const f32x4 hi = *reinterpret_cast<const f32x4 *>(row + ks * 32 + kq * 8 + 4);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                xr[g][ks][t] = agpr_put(lo[t]);
-                xr[g][ks][4 + t] = agpr_put(hi[t]);
+                for (int p = u * KS; p < (u + 1) * KS && p < R; ++p) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    ring[p] = load_a(cbx, p / KS, p % KS);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-    }
+    };
+    if (kEarly) fill(c.cbx, c.a.nhh);
 
     for (int s = 0; s < c.a.Q; ++s) {
         const StageArgs a = cascade_stage(c, s, K);
-        // ---- fp16 fragments and rounding norms of the residual ----
-        u32x4 xb[FG][KS];
-        float nx2[FG], nd2[FG], nxx2[FG];
+        const uint16_t *cbx = c.cbx + static_cast<int64_t>(s) * N * K;
+        if (!kEarly) fill(cbx, a.nhh);
+        __syncthreads();   // the residual rows are in place
+        // ---- fp16 fragments and rounding norms ----
+        for (int ks = wave; ks < KS; ks += kNwWaves) {
 #pragma unroll
-        for (int g = 0; g < FG; ++g) {
-            float sx = 0.0f, sd = 0.0f, sxx = 0.0f;
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                float v[8];
-#pragma unroll
-                for (int t = 0; t < 8; ++t) v[t] = agpr_get(xr[g][ks][t]);
+            for (int g = 0; g < FG; ++g) {
+                const float *row = xr + (g * 16 + col) * LY::XSTR + ks * 32 + kq * 8;
+                const f32x4 lo = *reinterpret_cast<const f32x4 *>(row), hi = *reinterpret_cast<const f32x4 *>(row + 4);
+                float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
                 // a Q8_0 codebook scores the query's Q8_0 image (as the sweep)
-                if (Q8) q8_image_block(v);
+                if (Q8) {
+                    const int f = g * 16 + col;
+                    q8_image_block(v, xq + f * LY::XQS + ks * 32 + kq * 8, xd + f * KS + ks);
+                }
                 u32x4 packed;
+                float sx = 0.0f, sd = 0.0f, sxx = 0.0f;
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const float v0 = v[2 * t], v1 = v[2 * t + 1];
@@ -3444,183 +3552,158 @@ __global__ __launch_bounds__(kRsThreads, 1) void euclid_resident_kernel(CascadeA
                     sxx = __fmaf_rn(v0, v0, sxx);
                     sxx = __fmaf_rn(v1, v1, sxx);
                 }
-                xb[g][ks] = packed;
+                xh[(g * KS + ks) * kWave + lane] = packed;
+                sx = rows_sum(sx);
+                sd = rows_sum(sd);
+                sxx = rows_sum(sxx);
+                if (kq == 0) {
+                    float *n3 = nrm + ks * 3 * LY::FRAMES + g * 16 + col;
+                    n3[0] = sx;
+                    n3[LY::FRAMES] = sd;
+                    n3[2 * LY::FRAMES] = sxx;
+                }
             }
-            sx = rows_sum(sx);
-            sd = rows_sum(sd);
-            sxx = rows_sum(sxx);
-            nx2[g] = sx;
-            nd2[g] = sd;
-            nxx2[g] = sxx;
         }
-
-        // ---- sweep of the stage's codebook ----
-        float top[FG][TOPL];
+        __syncthreads();
+        typename MX::V8 xb[FG][KS];
 #pragma unroll
         for (int g = 0; g < FG; ++g)
 #pragma unroll
-            for (int j = 0; j < TOPL; ++j) top[g][j] = -INFINITY;
-        auto lds_a = [&](int buf, int blk, int ks) -> typename MX::V8 {
-            const int r = blk * 16 + col;
-            const int j = ks * 4 + kq;
-            return *reinterpret_cast<const typename MX::V8 *>(lds + buf * LY::BUFB + r * T::ROWB + ((j ^ (r & T::SWZ)) * 16));
-        };
-        auto lds_h = [&](int buf, int blk) -> f32x4 {
-            return *reinterpret_cast<const f32x4 *>(lds + buf * LY::BUFB + T::CHUNKB + (blk * 16 + kq * 4) * 4);
-        };
-        // direct global-to-LDS staging, as in the sweep kernel (lane l of
-        // wave w lands at piece k * kRsThreads + 64 w + l)
-        const unsigned char *cbb = reinterpret_cast<const unsigned char *>(a.cbh);
-        auto stage_piece = [&](int buf, int chunk, int k) {
-            const unsigned char *gp = cbb + (static_cast<int64_t>(chunk) * T::CHUNKB + so.uni(k)) + so.lane(k);
-            unsigned char *d = lds + buf * LY::BUFB + (k * kRsThreads + wave * kWave) * 16;
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)gp,
-                                             (__attribute__((address_space(3))) void *)d, 16, 0, 0);
-        };
-        auto stage_h = [&](int buf, int chunk) {
-            const float *gp = a.nhh + static_cast<int64_t>(chunk) * T::CC + hsrc;
-            unsigned char *d = lds + buf * LY::BUFB + T::CHUNKB + wave * kWave * 4;
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)gp,
-                                             (__attribute__((address_space(3))) void *)d, 4, 0, 0);
-        };
-        __syncthreads();   // the previous stage's select is done with the scratch
-#pragma unroll
-        for (int k = 0; k < LY::STAGE16; ++k) stage_piece(0, 0, k);
-        stage_h(0, 0);
-        __builtin_amdgcn_s_waitcnt(kWaitLoads);
-        __syncthreads();
+            for (int ks = 0; ks < KS; ++ks) xb[g][ks] = __builtin_bit_cast(typename MX::V8, xh[(g * KS + ks) * kWave + lane]);
 
-        typename MX::V8 ring[R];
+        // sum_rows(x*x), a lane per frame: 256 dependent additions that the
+        // wave's SIMD partner sweeps beside
+        if (RECIPE == HIGGS && wave < FG && lane < 16)
+            x2s[wave * 16 + lane] = sum_squares_k<K>(xr + (wave * 16 + lane) * LY::XSTR);
+
+        // ---- this wave's codes ----
+        float top[FG][TS];
 #pragma unroll
-        for (int l = 0; l < L; ++l) ring[l] = lds_a(0, 0, l);
-        f32x4 hcur = lds_h(0, 0);
-        f32x4 accp[FG];
+        for (int g = 0; g < FG; ++g)
 #pragma unroll
-        for (int g = 0; g < FG; ++g) accp[g] = f32x4{-3.40282347e38f, -3.40282347e38f, -3.40282347e38f, -3.40282347e38f};
-        unsigned lprev = 0;
-        // key e (< 4 FG) of the previous block's sums into its group's list
-        auto insert_key = [&](const f32x4 (&acc)[FG], unsigned local0, int e) {
-            const int g = e / 4, i = e % 4;
-            const float key = key_of(acc[g][i], local0 + i, vkeep);
+            for (int j = 0; j < TS; ++j) top[g][j] = -INFINITY;
+        auto insert_keys = [&](const f32x4 (&acc)[FG], unsigned local0) {
 #pragma unroll
-            for (int j = TOPL - 1; j > 0; --j) top[g][j] = __builtin_amdgcn_fmed3f(top[g][j - 1], top[g][j], key);
-            top[g][0] = __builtin_amdgcn_fmed3f(top[g][0], key, 3.40282347e38f);
-        };
-        constexpr int E = 4 * FG;   // keys per block and lane
-        for (int ch = 0; ch < nch; ++ch) {
-            const int buf = ch & 1;
-            const int cs = ch + 1 < nch ? ch + 1 : ch;   // the last chunk re-stages itself (no branch)
+            for (int i = 0; i < 4; ++i) {
+                // in a scalar register of its own, so that the key is one
+                // v_and_or_b32
+                unsigned local = local0 + i;
+                asm("" : "+s"(local));
 #pragma unroll
-            for (int b = 0; b < BPC; ++b) {
+                for (int g = 0; g < FG; ++g) {
+                    const float key = key_of(acc[g][i], local, vkeep);
 #pragma unroll
-                for (int j = 0; j < PPB; ++j) {
-                    const int k = b + j * BPC;
-                    if (k < LY::STAGE16) stage_piece(buf ^ 1, cs, k);
+                    for (int j = TS - 1; j > 0; --j) top[g][j] = __builtin_amdgcn_fmed3f(top[g][j - 1], top[g][j], key);
+                    top[g][0] = __builtin_amdgcn_fmed3f(top[g][0], key, 3.40282347e38f);
                 }
-                if (b == 0) stage_h(buf ^ 1, cs);
-                const f32x4 hnext = b + 1 < BPC ? lds_h(buf, b + 1) : hcur;
+            }
+        };
+        for (int i0 = 0; i0 < nb; i0 += U) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
                 f32x4 acc[FG];
 #pragma unroll
-                for (int g = 0; g < FG; ++g) acc[g] = hcur;
-                // One wave per SIMD hides no latency behind another wave:
-                // scheduling barriers keep each step's fragment load L steps
-                // ahead of its MFMAs (the compiler would sink it next to
-                // them), and each step takes its share of the previous
-                // block's keys.
+                for (int g = 0; g < FG; ++g) acc[g] = hring[u];
+                hring[u] = load_h(a.nhh, i0 + u + U);
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
-                    const int pk = ks + L;
-                    if (pk < KS) ring[pk % R] = lds_a(buf, b, pk);
-                    else if (b + 1 < BPC) ring[pk % R] = lds_a(buf, b + 1, pk - KS);
-                    __builtin_amdgcn_sched_barrier(0);
+                    const int p = u * KS + ks;
 #pragma unroll
-                    for (int g = 0; g < FG; ++g)
-                        acc[g] = MX::mfma(ring[ks % R], __builtin_bit_cast(typename MX::V8, xb[g][ks]), acc[g]);
-#pragma unroll
-                    for (int e = ks * E / KS; e < (ks + 1) * E / KS; ++e) insert_key(accp, lprev, e);
+                    for (int g = 0; g < FG; ++g) acc[g] = MX::mfma(ring[p % R], xb[g][ks], acc[g]);
+                    ring[p % R] = load_a(cbx, i0 + (p + R) / KS, (p + R) % KS);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-#pragma unroll
-                for (int g = 0; g < FG; ++g) accp[g] = acc[g];
-                hcur = hnext;
-                lprev = static_cast<unsigned>((ch * BPC + b) * 4);
+                if (i0 + u < nb) insert_keys(acc, static_cast<unsigned>(wave + kNwWaves * (i0 + u)) * 4);   // wave-uniform
             }
-            __builtin_amdgcn_s_waitcnt(kWaitLoads);
-            __syncthreads();
-#pragma unroll
-            for (int l = 0; l < L; ++l) ring[l] = lds_a(buf ^ 1, 0, l);
-            hcur = lds_h(buf ^ 1, 0);
         }
 #pragma unroll
-        for (int e = 0; e < E; ++e) insert_key(accp, lprev, e);
-        __syncthreads();   // every wave is done with the chunk buffers
+        for (int g = 0; g < FG; ++g)
+#pragma unroll
+            for (int j = 0; j < TS; ++j) keys[((wave * FG + g) * TS + j) * kWave + lane] = top[g][j];
+        __syncthreads();
 
-        // ---- select and residual update of the wave's groups ----
-        unsigned char *ws = lds + wave * LY::WSCR;
-        SelLds<Q8, K, TOPL> &sl = *reinterpret_cast<SelLds<Q8, K, TOPL> *>(ws);
-        float *xs = reinterpret_cast<float *>(ws + LY::SELB);
+        // ---- merge, select and residual update of this wave's frames ----
+        const int g = wave / WPG, f0 = wave % WPG * FPW;
+        const int64_t mb = m_tile + g * 16;
+        float mt[TOPL], taul = -INFINITY;
 #pragma unroll
-        for (int g = 0; g < FG; ++g) {
-            const int64_t mb = m_wave + g * 16;
-            if (mb >= M) break;   // wave-uniform; later groups are further on
-            // the group's rows, for the exact re-ranking
+        for (int j = 0; j < TOPL; ++j) mt[j] = -INFINITY;
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                float *d = xs + col * LY::XSTR + ks * 32 + kq * 8;
-                *reinterpret_cast<f32x4 *>(d) = f32x4{agpr_get(xr[g][ks][0]), agpr_get(xr[g][ks][1]),
-                                                      agpr_get(xr[g][ks][2]), agpr_get(xr[g][ks][3])};
-                *reinterpret_cast<f32x4 *>(d + 4) = f32x4{agpr_get(xr[g][ks][4]), agpr_get(xr[g][ks][5]),
-                                                          agpr_get(xr[g][ks][6]), agpr_get(xr[g][ks][7])};
+        for (int w = 0; w < kNwWaves; ++w)
+#pragma unroll
+            for (int j = 0; j < TS; ++j) {
+                const float key = keys[((w * FG + g) * TS + j) * kWave + lane];
+                if (j == TS - 1) taul = fmaxf(taul, key);
+                // what the merged list drops bounds the rest too
+                taul = fmaxf(taul, fminf(mt[TOPL - 1], key));
+#pragma unroll
+                for (int i = TOPL - 1; i > 0; --i) mt[i] = __builtin_amdgcn_fmed3f(mt[i - 1], mt[i], key);
+                mt[0] = __builtin_amdgcn_fmed3f(mt[0], key, 3.40282347e38f);
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            const int code = select_group<RECIPE, Q8, KS, TOPL>(a, mb, top[g], top[g][TOPL - 1], nx2[g], nd2[g],
-                                                                   nxx2[g], sl, true, xs, LY::XSTR, false);
-            // r -= c[code] (the forced code where given) in registers
-            const int64_t m = mb + col;
-            int use = code >= 0 ? code : 0;
-            if (a.force_idx && m < M) {
-                use = a.force_idx[m * a.Q + s];
+        float n3[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            n3[q] = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) n3[q] += nrm[(ks * 3 + q) * LY::FRAMES + g * 16 + col];
+        }
+        __syncthreads();   // keys and fragments are read: the select queues take their place
+        SelLds<Q8, K, TOPL, true> &sl = *reinterpret_cast<SelLds<Q8, K, TOPL, true> *>(phase + wave * LY::SELB);
+        const bool update = s + 1 < a.Q || c.write_last;
+        const bool mine = mb + f0 < M;   // wave-uniform
+        float *xg = xr + g * 16 * LY::XSTR;
+        int use = 0;
+        if (mine) {
+            const int code = select_group<RECIPE, Q8, KS, TOPL, true>(
+                a, mb, mt, taul, n3[0], n3[1], n3[2], sl, true, xg, LY::XSTR, false, ((1u << FPW) - 1u) << f0,
+                SelPre{x2s + g * 16, xq + g * 16 * LY::XQS, xd + g * 16 * KS});
+            use = code >= 0 ? code : 0;
+            if (a.force_idx && code >= 0) {
+                use = a.force_idx[(mb + col) * a.Q + s];
                 if (use < 0 || use >= N) {
                     a.flags[AQ_FLAG_BAD_INDEX] = 1;
                     use = 0;
                 }
             }
-            if (s + 1 < a.Q || c.write_last) {
-                const float *crow = a.cbf + static_cast<int64_t>(use) * K;
-                f32x4 cv[KS][2];
+        }
+        // r -= c[code] (the forced code where given), rows across the lanes
+        f32x4 cv[KV][FPW];
+        if (mine && update) {
 #pragma unroll
-                for (int ks = 0; ks < KS; ++ks) {
-                    cv[ks][0] = *reinterpret_cast<const f32x4 *>(crow + ks * 32 + kq * 8);
-                    cv[ks][1] = *reinterpret_cast<const f32x4 *>(crow + ks * 32 + kq * 8 + 4);
+            for (int t = 0; t < FPW; ++t) {
+                const float *row = a.cbf + static_cast<int64_t>(__builtin_amdgcn_readlane(use, f0 + t)) * K;
+#pragma unroll
+                for (int kv = 0; kv < KV; ++kv) {
+                    const int k = (kv * kWave + lane) * 4;
+                    cv[kv][t] = *reinterpret_cast<const f32x4 *>(row + (k < K ? k : 0));
                 }
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-                    for (int t = 0; t < 8; ++t)
-                        xr[g][ks][t] = agpr_put(__fsub_rn(agpr_get(xr[g][ks][t]), cv[ks][t / 4][t % 4]));
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        if (kEarly && s + 1 < a.Q) fill(cbx + static_cast<int64_t>(N) * K, a.nhh + N);
+        if (mine && update) {
+#pragma unroll
+            for (int t = 0; t < FPW; ++t)
+#pragma unroll
+                for (int kv = 0; kv < KV; ++kv) {
+                    const int k = (kv * kWave + lane) * 4;
+                    if (k < K) {
+                        f32x4 *d = reinterpret_cast<f32x4 *>(xg + (f0 + t) * LY::XSTR + k);
+                        f32x4 o = *d;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) o[q] = __fsub_rn(o[q], cv[kv][t][q]);
+                        *d = o;
+                    }
+                }
         }
     }
 
     // the residual after the last stage
     if (c.write_last) {
-#pragma unroll
-        for (int g = 0; g < FG; ++g) {
-            const int64_t m = m_wave + g * 16 + col;
-            if (m >= M) continue;
-            float *row = c.work + m * K;
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                *reinterpret_cast<f32x4 *>(row + ks * 32 + kq * 8) =
-                    f32x4{agpr_get(xr[g][ks][0]), agpr_get(xr[g][ks][1]), agpr_get(xr[g][ks][2]), agpr_get(xr[g][ks][3])};
-                *reinterpret_cast<f32x4 *>(row + ks * 32 + kq * 8 + 4) =
-                    f32x4{agpr_get(xr[g][ks][4]), agpr_get(xr[g][ks][5]), agpr_get(xr[g][ks][6]), agpr_get(xr[g][ks][7])};
-            }
+        __syncthreads();
+        for (int e = threadIdx.x; e < LY::FRAMES * (K / 4); e += kNwThreads) {
+            const int f = e / (K / 4), k = e % (K / 4) * 4;
+            if (m_tile + f < M)
+                *reinterpret_cast<f32x4 *>(c.work + (m_tile + f) * K + k) = *reinterpret_cast<const f32x4 *>(xr + f * LY::XSTR + k);
         }
     }
 }
@@ -3678,9 +3761,9 @@ __device__ inline bool same_bits(float x, float y) { return __float_as_uint(x) =
 template <int RECIPE, bool Q8, int KS>
 __device__ inline void scan_frame(const StageArgs &a, const float *xs, const int8_t *xq, const float *xd, ScanSh &sh) {
     constexpr int K = KS * 32;
-    constexpr bool kQuadOk = !Q8 && RECIPE != DIRECT;
+    constexpr bool kQuadOk = !Q8;
     if constexpr (kQuadOk) {
-        if (spread_quad<RECIPE, Q8>(a) && a.N <= kScanChunk) {
+        if (quad_form<RECIPE, Q8>(a) && a.N <= kScanChunk) {
             block_values_quad<RECIPE, K>(a, xs, sh.o_x2, sh.rv, 0, a.N);
             __syncthreads();
             scan_select<RECIPE, Q8, KS>(a, K, true, sh.rv, xs, xq, xd, sh.o_x2, sh);
@@ -3702,7 +3785,7 @@ __device__ inline void scan_frame(const StageArgs &a, const float *xs, const int
 // euclid_verify_values_kernel (into a.svals, up to a.scap pairs).
 template <int RECIPE, bool Q8>
 __device__ inline bool verify_spread(const StageArgs &a, int count) {
-    const bool form = Q8 ? RECIPE == HIGGS : RECIPE != DIRECT && spread_quad<RECIPE, Q8>(a);
+    const bool form = Q8 ? RECIPE == HIGGS : quad_form<RECIPE, Q8>(a);
     return form && count <= a.scap;
 }
 constexpr int kVerifyPart = 128;   // codes per item of euclid_verify_values_kernel
@@ -3713,7 +3796,7 @@ constexpr int kVerifyPart = 128;   // codes per item of euclid_verify_values_ker
 template <int RECIPE, bool Q8, int KS>
 __global__ __launch_bounds__(kScanThreads) void euclid_verify_values_kernel(CascadeArgs c) {
     constexpr int K = KS * 32;
-    constexpr bool kQuadOk = !Q8 && RECIPE != DIRECT;
+    constexpr bool kQuadOk = !Q8;
     if constexpr (kQuadOk || (Q8 && RECIPE == HIGGS)) {
         extern __shared__ __align__(16) unsigned char lds[];
         float *xs = reinterpret_cast<float *>(lds);
@@ -3858,25 +3941,6 @@ constexpr int cascade_lds_bytes() {
     if constexpr (KS == 2 || KS == 8) return CLayout<KS, groups_for(KS), 4, true>::BYTES;
     else return 0;
 }
-// Register-resident cascade: K = 256 (3 groups of fp32 residual and fp16
-// fragments per wave fit its 512 registers).  The Q8_0 variant for top-k
-// keeps six keys per lane in place of four: its fp16 images of q * d leave
-// about 2.7 % of the frames of each stage uncertified with four (their
-// verification then costs more than the cascade saves), a few with six.
-constexpr int kRsGroups = 3;
-template <bool Q8, int TOPL>
-constexpr int resident_keys() { return Q8 && TOPL == 4 ? 6 : TOPL; }
-template <int RECIPE, bool Q8, int KS, int TOPL>
-constexpr CascadeFn resident_fn() {
-    if constexpr (KS == 8) return euclid_resident_kernel<RECIPE, Q8, KS, kRsGroups, resident_keys<Q8, TOPL>()>;
-    else return nullptr;
-}
-template <int KS>
-constexpr int resident_lds_bytes() {   // the largest variant's (Q8_0, six keys)
-    if constexpr (KS == 8) return RsLayout<KS, kRsGroups, resident_keys<true, 4>(), true>::BYTES;
-    else return 0;
-}
-
 }  // namespace
 
 // Defines aq_euclid::kernels_ks<KS>(): the kernel table of one width.
@@ -3910,13 +3974,7 @@ constexpr int resident_lds_bytes() {   // the largest variant's (Q8_0, six keys)
             {fixup_fn<OMNI, false, KS>(), fixup_fn<HIGGS, false, KS>(), fixup_fn<DIRECT, false, KS>(),          \
              fixup_fn<HIGGS, true, KS>()},                                                                      \
             cascade_lds_bytes<KS>(),                                                                            \
-            kCRows * groups_for(KS) * 16,                                                                       \
-            {{resident_fn<OMNI, false, KS, 3>(), resident_fn<OMNI, false, KS, 4>()},                            \
-             {resident_fn<HIGGS, false, KS, 3>(), resident_fn<HIGGS, false, KS, 4>()},                          \
-             {resident_fn<DIRECT, false, KS, 3>(), resident_fn<DIRECT, false, KS, 4>()},                        \
-             {resident_fn<HIGGS, true, KS, 3>(), resident_fn<HIGGS, true, KS, 4>()}},                           \
-            resident_lds_bytes<KS>(),                                                                           \
-            kRsWaves * kRsGroups * 16};                                                                         \
+            kCRows * groups_for(KS) * 16};                                                                      \
         return &t;                                                                                              \
     }                                                                                                           \
     }

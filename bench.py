@@ -200,9 +200,9 @@ class EuclidRvq:
 
     def one_launch(self):
         """The step ran as one timed launch for all stages: the one-launch
-        cascade (register-resident at K = 256)."""
+        cascade (residual in LDS at K = 256)."""
         self.stages_per_launch = self.Q
-        self.kernel = "euclid_resident_kernel" if self.K == 256 else "euclid_cascade_kernel"
+        self.kernel = "euclid_narrow_kernel" if self.K == 256 else "euclid_cascade_kernel"
 
     def flops_per_launch(self) -> float:
         # the distance contraction of one stage is 2 * N * K per frame

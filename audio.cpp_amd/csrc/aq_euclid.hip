@@ -525,6 +525,19 @@ aq_status aq_euclid_upload_projected(aq_ctx *ctx, int64_t Q, int64_t N, int64_t 
     }
     aq_device_guard g(ctx->device);
     st = aq_proj_create(ctx, Q, N, K, H, cb->d_cbf, proj_type, w_in, b_in, w_out, b_out, &cb->proj);
+    if (st == AQ_OK) st = aq_proj_cascade_weights(ctx, cb->proj);
+    if (st == AQ_OK && cb->proj->w_cx && !cb->d_cbx) {   // the cascade's codebook image
+        const int64_t pieces = Q * N * K / 8;
+        if (hipMalloc(&cb->d_cbx, static_cast<size_t>(pieces) * 16) != hipSuccess) {
+            st = aq_fail(ctx, AQ_E_NOMEM, "aq_euclid_upload: device allocation failed");
+        } else {
+            hipLaunchKernelGGL(euclid_fragments_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
+                               ctx->stream, reinterpret_cast<const u32x4 *>(cb->d_cbh), pieces, static_cast<int>(K),
+                               reinterpret_cast<u32x4 *>(cb->d_cbx));
+            if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess)
+                st = aq_fail(ctx, AQ_E_DEVICE, "aq_euclid_upload_projected: codebook image failed");
+        }
+    }
     if (st != AQ_OK) {
         aq_euclid_release(cb);
         return st;
@@ -617,6 +630,15 @@ aq_status noalloc_region(aq_ctx *ctx, unsigned char **out) {
     return AQ_OK;
 }
 
+// Whether a forced code was out of range (synchronises the stream).
+aq_status check_forced(aq_ctx *ctx, const aq_codebooks *cb) {
+    int32_t flag = 0;
+    AQ_HIP(ctx, hipMemcpyAsync(&flag, ctx->d_flags + AQ_FLAG_BAD_INDEX, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+    AQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (flag) return aq_fail(ctx, AQ_E_INDEX_RANGE, "aq_euclid_encode: force_idx holds a code outside [0, %lld)", (long long)cb->N);
+    return AQ_OK;
+}
+
 // Encode on an any-width codebook set: per stage, the exact scan of every
 // frame in the recipe's arithmetic (the run-time-width exact scan, one block
 // per frame), with the residual cascade r -= c[code] in between.
@@ -681,13 +703,7 @@ aq_status euclid_encode_any(aq_ctx *ctx, const aq_codebooks *cb, const aq_frames
         aq_launch_timed(ctx, !arena.base, scan, dim3(grid), dim3(kScanThreads), static_cast<uint32_t>(lds), a);
         AQ_HIP(ctx, hipGetLastError());
     }
-    if (force_idx) {
-        int32_t flag = 0;
-        AQ_HIP(ctx, hipMemcpyAsync(&flag, ctx->d_flags + AQ_FLAG_BAD_INDEX, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
-        AQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (flag) return aq_fail(ctx, AQ_E_INDEX_RANGE, "aq_euclid_encode: force_idx holds a code outside [0, %lld)", (long long)cb->N);
-    }
-    return AQ_OK;
+    return force_idx ? check_forced(ctx, cb) : AQ_OK;
 }
 
 // The encode pipeline of a plain codebook: the narrow one-launch cascade
@@ -856,13 +872,48 @@ aq_status euclid_encode_cascade(aq_ctx *ctx, const aq_codebooks *cb, const aq_fr
     AQ_HIP(ctx, hipGetLastError());
     hipLaunchKernelGGL(fix, dim3(static_cast<unsigned>(cus)), dim3(kScanThreads), slds, ctx->stream, c);
     AQ_HIP(ctx, hipGetLastError());
-    if (force_idx) {
-        int32_t flag = 0;
-        AQ_HIP(ctx, hipMemcpyAsync(&flag, ctx->d_flags + AQ_FLAG_BAD_INDEX, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
-        AQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (flag) return aq_fail(ctx, AQ_E_INDEX_RANGE, "aq_euclid_encode: force_idx holds a code outside [0, %lld)", (long long)cb->N);
-    }
-    return AQ_OK;
+    return force_idx ? check_forced(ctx, cb) : AQ_OK;
+}
+
+// A projected encode in one launch (aq_proj_cascade).  The exact scans of
+// open frames happen in the block, so both counters of a stage are those
+// frames.
+aq_status euclid_encode_projected(aq_ctx *ctx, const aq_codebooks *cb, const aq_frames_desc &in, int64_t M, int32_t *idx,
+                                  float *residual, float *dist, int topk, int32_t *topk_idx, float *topk_dist,
+                                  const int32_t *force_idx, Arena &arena, int topl) {
+    int32_t *counts = nullptr;
+    aq_status st = arena.get(1, 128 * sizeof(int32_t), reinterpret_cast<void **>(&counts));
+    if (st != AQ_OK) return st;
+    ctx->euclid_counts = counts;
+    hipLaunchKernelGGL(zero2_kernel, dim3(1), dim3(256), 0, ctx->stream, counts, 128, ctx->d_flags,
+                       static_cast<int>(AQ_FLAG_COUNT));
+    AQ_HIP(ctx, hipGetLastError());
+    CascadeArgs c{};
+    StageArgs &a = c.a;
+    a.M = M;
+    a.N = static_cast<int>(cb->N);
+    a.K = static_cast<int>(cb->K);
+    a.cbh = cb->d_cbh;
+    a.nhh = cb->d_hh;
+    a.cbf = cb->d_cbf;
+    a.bias = cb->d_bias;
+    a.e2 = cb->d_e2;
+    a.q8 = cb->q8 ? cb->d_q8 : nullptr;
+    a.q8d = cb->q8 ? cb->d_q8d : nullptr;
+    a.Q = static_cast<int>(cb->Q);
+    a.idx = idx;
+    a.dist = dist;
+    a.topk = topk;
+    a.topk_idx = topk_idx;
+    a.topk_dist = topk_dist;
+    a.flags = ctx->d_flags;
+    a.exact_only = cb->exact_only ? 1 : 0;
+    c.cbx = cb->d_cbx;
+    c.bounds = cb->d_bounds;
+    c.counts = counts;
+    st = aq_proj_cascade(ctx, cb->proj, c, cb->q8, cb->recipe, topl, in, force_idx, residual, !arena.base);
+    if (st != AQ_OK) return st;
+    return force_idx ? check_forced(ctx, cb) : AQ_OK;
 }
 
 // Encode M frames (strided input `in`) through every stage of cb.  Plain
@@ -901,6 +952,15 @@ aq_status euclid_encode_impl(aq_ctx *ctx, const aq_codebooks *cb, const aq_frame
     if (pipe != Pipeline::kStages)
         return euclid_encode_cascade(ctx, cb, in, M, idx, residual, dist, topk, topk_idx, topk_dist, force_idx, arena, kk,
                                      var, topl, pipe, fg);
+    // Projected cascades at K = 64 run in one launch (8 stages at 250
+    // frames 89 us, per stage 699; 6 000 frames with Q8_0 weights 348 us, per
+    // stage 1 415).  Calls from the
+    // fixed region keep the per-stage launches and their limits;
+    // AQ_EUCLID_PIPELINE=stages asks for them too (comparisons and tests).
+    const char *pipe_env = std::getenv("AQ_EUCLID_PIPELINE");
+    if (pw && !arena.base && cb->d_cbx && aq_proj_cascade_shape(pw, cb->N, M) &&
+        !(pipe_env && std::strcmp(pipe_env, "stages") == 0))
+        return euclid_encode_projected(ctx, cb, in, M, idx, residual, dist, topk, topk_idx, topk_dist, force_idx, arena, topl);
     StageFn sweep = kk->sweep[cb->q8 ? 1 : 0][topl - 3];
     StageFn select = kk->select[var][topl - 3];
     StageFn scan = kk->exact_scan[var];
@@ -1170,13 +1230,7 @@ aq_status euclid_encode_impl(aq_ctx *ctx, const aq_codebooks *cb, const aq_frame
             if (st != AQ_OK) return st;
         }
     }
-    if (force_idx) {
-        int32_t flag = 0;
-        AQ_HIP(ctx, hipMemcpyAsync(&flag, ctx->d_flags + AQ_FLAG_BAD_INDEX, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
-        AQ_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (flag) return aq_fail(ctx, AQ_E_INDEX_RANGE, "aq_euclid_encode: force_idx holds a code outside [0, %lld)", (long long)cb->N);
-    }
-    return AQ_OK;
+    return force_idx ? check_forced(ctx, cb) : AQ_OK;
 }
 
 }  // namespace

@@ -511,7 +511,7 @@ void aq_proj_release(aq_proj_weights *pw) {
     if (!pw) return;
     for (void *p : {static_cast<void *>(pw->w_in), static_cast<void *>(pw->w_in_q), static_cast<void *>(pw->w_in_d),
                     static_cast<void *>(pw->b_in), static_cast<void *>(pw->w_out), static_cast<void *>(pw->b_out),
-                    static_cast<void *>(pw->table)})
+                    static_cast<void *>(pw->table), pw->w_cx})
         if (p) (void)hipFree(p);
     delete pw;
 }

@@ -28,6 +28,7 @@ struct aq_proj_weights {
     int8_t *w_in_q = nullptr;   // [Q][K][H] quants (Q8_0)
     float *w_in_d = nullptr;    // [Q][K][H/32] scales (Q8_0)
     float *b_in = nullptr;      // [Q][K] or null
+    void *w_cx = nullptr;       // project_in in the one-launch cascade's layout (K = 64)
     float *w_out = nullptr;     // [Q][H][K] (F32; the single-frame path)
     float *b_out = nullptr;     // [Q][H] or null
     float *table = nullptr;     // [Q][N][H]: project_out(c[n]) + b_out
@@ -70,6 +71,17 @@ aq_status aq_proj_decode(aq_ctx *ctx, const aq_proj_weights *pw, const int32_t *
 // fits a CU next to their static LDS; else AQ_E_SHAPE with `fn` in the
 // message.
 aq_status aq_proj_check_lds(aq_ctx *ctx, int64_t H, bool q8, const char *fn);
+
+// The one-launch projected cascade (aq_projected_cascade.hip): whether its
+// kernels take the shape, its weight images (at upload), and the encode of
+// c's frames through every stage (c: stage 0's codebook pointers, bounds,
+// counts and outputs; force: the update's codes or null; rout [M, H] or
+// null).
+namespace aq_euclid { struct CascadeArgs; }
+bool aq_proj_cascade_shape(const aq_proj_weights *pw, int64_t N, int64_t M);
+aq_status aq_proj_cascade_weights(aq_ctx *ctx, aq_proj_weights *pw);
+aq_status aq_proj_cascade(aq_ctx *ctx, const aq_proj_weights *pw, const aq_euclid::CascadeArgs &c, bool q8c, int recipe,
+                          int topl, const aq_frames_desc &in, const int32_t *force, float *rout, bool timed);
 
 // Gather of a strided input into frame-major rows: out[m, c] for c < C.
 aq_status aq_gather_frames(aq_ctx *ctx, const aq_frames_desc &in, int64_t M, int64_t C, float *out);

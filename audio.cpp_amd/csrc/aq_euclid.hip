@@ -975,7 +975,7 @@ aq_status euclid_encode_impl(aq_ctx *ctx, const aq_codebooks *cb, const aq_frame
 
     // Sweep launch: tiles of kWaves * FG * 16 frames; the codebook is split
     // over blockIdx.y so that there are about two sweep waves per SIMD (each
-    // split a whole number of LDS chunks, at most 4 splits).
+    // split a whole number of LDS chunks, up to 4 splits).
     const int FG = groups_for(ks);
     const int64_t frames_per_block = static_cast<int64_t>(kWaves) * FG * 16;
     const int64_t tiles = (M + frames_per_block - 1) / frames_per_block;
@@ -984,6 +984,15 @@ aq_status euclid_encode_impl(aq_ctx *ctx, const aq_codebooks *cb, const aq_frame
     int nsplit = 1;
     for (int sp = 1; sp <= 4; ++sp)
         if (nch % sp == 0 && tiles * sp <= 2 * cus) nsplit = sp;
+    // Few tiles leave most CUs idle at 4 splits: more, while a block per CU is
+    // enough for all and a split keeps 128 codes.  K = 768, N = 16 384, 1 499
+    // frames (8 tiles): 4, 8, 16, 32 splits 358, 235, 176, 153 us, 64 (two
+    // blocks per CU) 194; 6 000 frames (32 tiles): 360, 241, 271, 346; N =
+    // 1 024, 200 frames: 76, 69 at 8 (128 codes), 70 at 32.  The fixed region
+    // of the no-allocation entry point keeps the keys of 4.
+    if (!arena.base)
+        for (int sp : {8, 16, 32})
+            if (nch % sp == 0 && tiles * sp <= cus && cb->N / sp >= 128) nsplit = sp;
     int nsplit2 = nsplit;
     int64_t tile2 = tiles8;   // no second part
     // Grids of several rounds of blocks: the tiles that fill whole rounds

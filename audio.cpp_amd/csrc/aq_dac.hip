@@ -288,15 +288,21 @@ __device__ __forceinline__ void project_frames(const float (&r)[FW][DI], const f
         for (int f = 0; f < FW; ++f)
 #pragma unroll
             for (int j = 0; j < 8; ++j) acc[f][j] = 0.0f;
-        // Weights are loaded one step ahead.
-        float4 wa = win[lane];
-        float4 wb = win[kWave + lane];
+        // Weights are loaded one step ahead (a wave of one frame has an eighth
+        // of the LDS latency's work in a step: four).
+        constexpr int AH = FW == 1 && DI >= 4 ? 4 : 1;
+        float4 ra[AH], rb[AH];
+#pragma unroll
+        for (int i = 0; i < AH; ++i) {
+            ra[i] = win[(i * 2 + 0) * kWave + lane];
+            rb[i] = win[(i * 2 + 1) * kWave + lane];
+        }
 #pragma unroll
         for (int i = 0; i < DI; ++i) {
-            float4 na = wa, nb = wb;
-            if (i + 1 < DI) {
-                na = win[((i + 1) * 2 + 0) * kWave + lane];
-                nb = win[((i + 1) * 2 + 1) * kWave + lane];
+            const float4 wa = ra[i % AH], wb = rb[i % AH];
+            if (i + AH < DI) {
+                ra[i % AH] = win[((i + AH) * 2 + 0) * kWave + lane];
+                rb[i % AH] = win[((i + AH) * 2 + 1) * kWave + lane];
             }
 #pragma unroll
             for (int f = 0; f < FW; ++f) {
@@ -310,8 +316,6 @@ __device__ __forceinline__ void project_frames(const float (&r)[FW][DI], const f
                 acc[f][6] = __fmaf_rn(v, wb.z, acc[f][6]);
                 acc[f][7] = __fmaf_rn(v, wb.w, acc[f][7]);
             }
-            wa = na;
-            wb = nb;
             // Pin this step's accumulators here: otherwise LLVM sinks the
             // later frames' FMA chains below the first frame's reduction and
             // keeps every step's weights live.
@@ -568,7 +572,10 @@ __global__ __launch_bounds__(kMaxBlock, 1) void dac_encode_kernel(
             k1[f] = -INFINITY;
             k2[f] = -INFINITY;
         }
-#pragma unroll 2
+        // codes' loads ahead of their keys: a wave of one frame does too little
+        // per code to cover the latency two at a time
+        constexpr int UC = FW > 1 ? 2 : (ORDER == 1 ? 4 : 8);
+#pragma unroll UC
         for (int c = 0; c < NC; ++c) {
             const float4 a = chat[(c * 2 + 0) * kWave + lane];
             const float4 b = chat[(c * 2 + 1) * kWave + lane];
@@ -1163,14 +1170,18 @@ using EncodeFn = void (*)(const float *, int64_t, int, int, const float4 *, int6
                           float *, float *, const int32_t *, int32_t *, int, int, float, int, float, int64_t, int, int);
 
 constexpr int kPrefetch = 12;   // float4 per thread in the prefetching variant
+// ... and of waves with one frame, whose registers have room (not with the
+// recon rows and the tinyBLAS order's): blocks of 4 waves hold the next image
+// of D = N = 1 024 too.  Eight stages of 647 frames 61 us without.
+constexpr int prefetch_of(int fw, bool recon, int order) { return fw == 1 && !(recon && order == 1) ? 17 : kPrefetch; }
 
 // Variants: image copied at each stage start, prefetched a stage ahead, or
 // (large codebooks) the W_in + b_in prefix prefetched with c_hat in memory.
 // ORDER: the in-projection's summation order, 0 ggml_vec_dot_f32, 1 tinyBLAS.
 template <int DI, int FW, bool RECON, int ORDER>
 EncodeFn pick_pf(bool prefetch, bool cbg) {
-    if (cbg) return dac_encode_kernel<DI, FW, RECON, kPrefetch, true, ORDER>;
-    return prefetch ? dac_encode_kernel<DI, FW, RECON, kPrefetch, false, ORDER>
+    if (cbg) return dac_encode_kernel<DI, FW, RECON, prefetch_of(FW, RECON, ORDER), true, ORDER>;
+    return prefetch ? dac_encode_kernel<DI, FW, RECON, prefetch_of(FW, RECON, ORDER), false, ORDER>
                     : dac_encode_kernel<DI, FW, RECON, 0, false, ORDER>;
 }
 
@@ -1260,7 +1271,7 @@ Shape launch_shape(int64_t M, int64_t D, int64_t img_f4, bool recon, int num_cus
         if (env_fw >= 1 && env_fw <= 3 && fw != env_fw) continue;
         for (int wpb : {4, 6, 8}) {
             if (env_wpb && wpb != env_wpb) continue;
-            bool prefetch = (img_f4 + wpb * kWave - 1) / (wpb * kWave) <= kPrefetch;
+            bool prefetch = (img_f4 + wpb * kWave - 1) / (wpb * kWave) <= prefetch_of(fw, recon, order);
             if (const char *e = std::getenv("AQ_DAC_PF")) prefetch = prefetch && std::atoi(e) != 0;
             if (cbg && !prefetch) continue;   // the in-memory codebook variant always prefetches
             hipFuncAttributes attr{};

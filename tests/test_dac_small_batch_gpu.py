@@ -1,0 +1,69 @@
+"""GPU parity of the DAC cascade at batches of one frame per wave: 4-wave
+blocks whose threads hold the next stage's image (D = N = 1 024: the last
+piece is a partial one), codebook chunks that are no multiple of the unrolled
+step, a codebook read from memory, both summation orders, with and without
+the reconstruction; channel-major input with ragged tiles; bit for bit."""
+
+import numpy as np
+import pytest
+
+from test_dac_gpu import _sha
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,D,N,channel_major,recon", [
+    (1, 1024, 1024, False, False),
+    (647, 1024, 1024, True, False),    # 162 blocks of 4 waves; the gather's last tile of 7 frames
+    (65, 1024, 960, True, True),       # 15 chunks of codes
+    (64, 1024, 1024, False, True),     # tinyBLAS order with recon: the copied image
+    (132, 1024, 1024, True, False),    # tinyBLAS order, held image
+    (5, 1024, 4096, False, False),     # codebook in memory
+    (63, 256, 64, True, True),
+])
+def test_dac_one_frame_per_wave(monkeypatch, T, D, N, channel_major, recon):
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import aqmi
+    from aqmi import synth
+    from oracle import Oracle
+
+    print(f"[gpu] dac one frame per wave T={T} D={D} N={N} cm={channel_major} recon={recon}", flush=True)
+    monkeypatch.setenv("AQ_DAC_FW", "1")
+    monkeypatch.setenv("AQ_DAC_WPB", "4")
+    Q = 3
+    cfg = dict(synth.dac_weights(91, Q, D, N, bias=True), x=synth.normal(91, 1, (T, D)), M=T, T=T, B=1, D=D, N=N, Q=Q)
+    st = aqmi.DacStages(aqmi.Context(0), cfg["w_in"], cfg.get("b_in"), cfg["codebook"], cfg["w_out"], cfg.get("b_out"))
+    x = torch.from_numpy(cfg["x"]).cuda()
+    x = x.t().contiguous() if channel_major else x
+    idx = torch.full((T, Q), -1, dtype=torch.int32, device="cuda")
+    res = torch.empty((T, D), dtype=torch.float32, device="cuda")
+    rec = torch.empty((T, D), dtype=torch.float32, device="cuda") if recon else None
+    st.encode_ex(x, T, T, (D * T, 1, T) if channel_major else (D * T, D, 1), idx.data_ptr(), Q, res, rec)
+    torch.cuda.synchronize()
+    ref = Oracle().dac_rvq(cfg)
+    assert np.array_equal(idx.cpu().numpy(), ref["idx"])
+    assert _sha(res.cpu().numpy()) == _sha(ref["residual"])
+    if recon:
+        assert _sha(rec.cpu().numpy()) == _sha(ref["recon"])
+
+
+@pytest.mark.parametrize("M", [9, 2049, 5121])   # 2, 3 and 6 waves per block, the last one of one frame
+def test_outetts_waves_per_block(M):
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import aqmi
+    from aqmi import synth
+    from oracle import Oracle
+    from test_hostloop_gpu import run_outetts
+
+    print(f"[gpu] outetts waves per block M={M}", flush=True)
+    cfg = synth.outetts_config(M)
+    got = run_outetts(torch, aqmi.Context(0), cfg)
+    want = Oracle().outetts_rvq(cfg)
+    assert np.array_equal(got["idx"], want["idx"])
+    assert _sha(got["residual"]) == _sha(want["residual"])

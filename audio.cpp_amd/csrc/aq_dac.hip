@@ -963,14 +963,29 @@ __global__ void dac_decode_kernel(const int32_t *__restrict__ idx, int64_t ld, i
     const int64_t m = t / D;
     const int64_t d = t % D;
     float acc = accumulate ? out[t] : 0.0f;
-    for (int s = 0; s < Q; ++s) {
-        int32_t code = idx[m * ld + s];
-        if (code < 0 || code >= N) {
-            flags[AQ_FLAG_BAD_INDEX] = 1;
-            code = 0;
+    // Eight stages' codes, then their rows, at once (past the last stage: the
+    // last again, not added): one by one, each stage waited for its code and
+    // then for its row (1 291 frames of 8 stages: 12.3 us).
+    constexpr int B = 8;
+    for (int s0 = 0; s0 < Q; s0 += B) {
+        int32_t code[B];
+        float z[B];
+#pragma unroll
+        for (int k = 0; k < B; ++k) code[k] = idx[m * ld + (s0 + k < Q ? s0 + k : Q - 1)];
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            if (code[k] < 0 || code[k] >= N) {
+                flags[AQ_FLAG_BAD_INDEX] = 1;
+                code[k] = 0;
+            }
         }
-        const float z = tables[(static_cast<int64_t>(s) * N + code) * D + d];
-        acc = (s == 0 && !accumulate) ? z : __fadd_rn(acc, z);
+#pragma unroll
+        for (int k = 0; k < B; ++k)
+            z[k] = tables[(static_cast<int64_t>(s0 + k < Q ? s0 + k : Q - 1) * N + code[k]) * D + d];
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            if (s0 + k < Q) acc = (s0 + k == 0 && !accumulate) ? z[k] : __fadd_rn(acc, z[k]);
+        }
     }
     out[t] = acc;
 }

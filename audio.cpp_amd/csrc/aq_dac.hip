@@ -1187,7 +1187,9 @@ using EncodeFn = void (*)(const float *, int64_t, int, int, const float4 *, int6
 constexpr int kPrefetch = 12;   // float4 per thread in the prefetching variant
 // ... and of waves with one frame, whose registers have room (not with the
 // recon rows and the tinyBLAS order's): blocks of 4 waves hold the next image
-// of D = N = 1 024 too.  Eight stages of 647 frames 61 us without.
+// of D = N = 1 024 too.  Eight stages of 647 frames 61 us without, 29 with.
+// A codebook in memory has the smaller prefix to hold: 17 pieces' clamped
+// loads cost its single stage 13 us.
 constexpr int prefetch_of(int fw, bool recon, int order) { return fw == 1 && !(recon && order == 1) ? 17 : kPrefetch; }
 
 // Variants: image copied at each stage start, prefetched a stage ahead, or
@@ -1195,7 +1197,7 @@ constexpr int prefetch_of(int fw, bool recon, int order) { return fw == 1 && !(r
 // ORDER: the in-projection's summation order, 0 ggml_vec_dot_f32, 1 tinyBLAS.
 template <int DI, int FW, bool RECON, int ORDER>
 EncodeFn pick_pf(bool prefetch, bool cbg) {
-    if (cbg) return dac_encode_kernel<DI, FW, RECON, prefetch_of(FW, RECON, ORDER), true, ORDER>;
+    if (cbg) return dac_encode_kernel<DI, FW, RECON, kPrefetch, true, ORDER>;
     return prefetch ? dac_encode_kernel<DI, FW, RECON, prefetch_of(FW, RECON, ORDER), false, ORDER>
                     : dac_encode_kernel<DI, FW, RECON, 0, false, ORDER>;
 }
@@ -1286,7 +1288,7 @@ Shape launch_shape(int64_t M, int64_t D, int64_t img_f4, bool recon, int num_cus
         if (env_fw >= 1 && env_fw <= 3 && fw != env_fw) continue;
         for (int wpb : {4, 6, 8}) {
             if (env_wpb && wpb != env_wpb) continue;
-            bool prefetch = (img_f4 + wpb * kWave - 1) / (wpb * kWave) <= prefetch_of(fw, recon, order);
+            bool prefetch = (img_f4 + wpb * kWave - 1) / (wpb * kWave) <= (cbg ? kPrefetch : prefetch_of(fw, recon, order));
             if (const char *e = std::getenv("AQ_DAC_PF")) prefetch = prefetch && std::atoi(e) != 0;
             if (cbg && !prefetch) continue;   // the in-memory codebook variant always prefetches
             hipFuncAttributes attr{};

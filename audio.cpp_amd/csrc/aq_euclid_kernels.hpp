@@ -2748,6 +2748,9 @@ __device__ inline float wave_sum(float v) {
     return v;
 }
 
+// A value that every lane holds alike, in a scalar register.
+__device__ inline float wave_uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
+
 // Exact values of one frame's candidates cn[0 .. ncand), in exact_value_kq's
 // arithmetic, with several candidates per pass and coalesced row reads:
 //  * tinyBLAS order and DIRECT: a quad of lanes per candidate (quad_step);
@@ -2791,8 +2794,10 @@ __device__ void exact_values_frame(const StageArgs &a, const float *__restrict__
     } else if (Q8) {
         const int j = lane & 7, grp = lane >> 3;
         const int *xqi = reinterpret_cast<const int *>(xq) + j;
-        for (int c = grp; c < ncand; c += 8) {
-            const int n = cn[c];
+        const int nc = __builtin_amdgcn_readfirstlane(ncand);   // a scalar trip count, as above
+        for (int c0 = 0; c0 < nc; c0 += 8) {
+            const int c = c0 + grp;
+            const int n = cn[c < nc ? c : c0];
             const int *cq = reinterpret_cast<const int *>(a.q8 + static_cast<int64_t>(n) * K) + j;
             const float *cd = a.q8d + static_cast<int64_t>(n) * (K / 32);
             float acc = 0.0f;
@@ -2804,10 +2809,14 @@ __device__ void exact_values_frame(const StageArgs &a, const float *__restrict__
             acc = __fadd_rn(acc, __shfl_xor(acc, 4));
             acc = __fadd_rn(acc, __shfl_xor(acc, 2));
             acc = __fadd_rn(acc, __shfl_xor(acc, 1));
-            if (j == 0) cv[c] = __fsub_rn(__fsub_rn(__fmul_rn(acc, 2.0f), x2), a.e2[n]);
+            if (j == 0 && c < nc) cv[c] = __fsub_rn(__fsub_rn(__fmul_rn(acc, 2.0f), x2), a.e2[n]);
         }
     } else {
-        for (int c = lane; c < ncand; c += kWave) cv[c] = exact_value_kq<RECIPE, Q8, K>(a, x, cn[c], x2, xq, xd);
+        const int nc = __builtin_amdgcn_readfirstlane(ncand);
+        for (int c0 = 0; c0 < nc; c0 += kWave) {
+            const int c = c0 + lane;
+            if (c < nc) cv[c] = exact_value_kq<RECIPE, Q8, K>(a, x, cn[c], x2, xq, xd);
+        }
     }
 }
 
@@ -2818,8 +2827,8 @@ __global__ __launch_bounds__(kWave) void euclid_refine_select_kernel(StageArgs a
     __shared__ int cand_n[kRCand];
     __shared__ float cand_v[kRCand];
     __shared__ float keys_s[kRKeyLds];     // the frame's keys of every slice
-    __shared__ float xs[K];                // the frame (exact evaluation reads it here)
-    __shared__ int8_t xq[Q8 ? K : 4];      // its Q8_0 blocks
+    __shared__ __align__(16) float xs[K];             // the frame (exact evaluation reads it here, 16 bytes at a time)
+    __shared__ __align__(16) int8_t xq[Q8 ? K : 4];   // its Q8_0 blocks
     __shared__ float xd[Q8 ? K / 32 : 1];
     __shared__ float x2s;
     const int lane = threadIdx.x;
@@ -2867,7 +2876,7 @@ __global__ __launch_bounds__(kWave) void euclid_refine_select_kernel(StageArgs a
             sxx = __fmaf_rn(v, v, sxx);
         }
         const float nxh = sqrtf(wave_sum(sh)) * 1.0001f, nxl = sqrtf(wave_sum(sl)) * 1.0001f;
-        const float nxr = sqrtf(wave_sum(sr)) * 1.0001f, nxx2 = wave_sum(sxx);
+        const float nxr = sqrtf(wave_sum(sr)) * 1.0001f, nxx2 = wave_uniform(wave_sum(sxx));
         const float nxe = nxh + nxl + nxr;   // >= |x|
         // Bound E (v units) on |s(n) - S'(n)| for every code n: dropped split
         // terms, fp32 accumulation of 3K products from -|c|^2/2, the recipe's
@@ -2877,11 +2886,12 @@ __global__ __launch_bounds__(kWave) void euclid_refine_select_kernel(StageArgs a
         const float e_acc = (3 * K + 8) * u * mag;
         const float e_rec = (K + 16) * u * (nxe * a.cmax + nxe * nxe + a.cmax * a.cmax);
         const float vmax = mag + e_acc;
-        const float E = 1.02f * (e_split + e_acc + e_rec + 4.0f * u * vmax) + ldexpf(vmax, 6 - 23) + 1e-30f;
-        // ok and ncand are the same in every lane (a block is one wave, E
-        // comes from butterfly sums): in scalar registers, so that no branch
-        // or loop below works through the execution mask
-        ok = __builtin_amdgcn_readfirstlane(ok && (E < INFINITY) ? 1 : 0) != 0;
+        // What the branches and loops below depend on is the same in every
+        // lane (a block is one wave; E, tau and the T-th key come from
+        // butterflies): it goes through scalar registers, so that none of
+        // them works through the execution mask (see exact_values_frame).
+        const float E = wave_uniform(1.02f * (e_split + e_acc + e_rec + 4.0f * u * vmax) + ldexpf(vmax, 6 - 23) + 1e-30f);
+        ok = ok && E < INFINITY;
 
         // Keys of every slice: tau bounds every code a lane dropped; vT is
         // the T-th largest key (ties by position).
@@ -2913,17 +2923,22 @@ __global__ __launch_bounds__(kWave) void euclid_refine_select_kernel(StageArgs a
         float vT = -INFINITY;
         int ncand = 0;
         if (ok) {
-            for (int e = lane * kTopR + kTopR - 1; e < nk; e += kWave * kTopR) tau = fmaxf(tau, kp[e]);
+            for (int e0 = 0; e0 < nk; e0 += kWave * kTopR) {
+                const int e = e0 + lane * kTopR + kTopR - 1;
+                tau = fmaxf(tau, e < nk ? kp[e] : -INFINITY);
+            }
 #pragma unroll
             for (int off = 1; off < kWave; off <<= 1) tau = fmaxf(tau, __shfl_xor(tau, off));
+            tau = wave_uniform(tau);
             float pv = INFINITY;
             int pp = -1;
             for (int t = 0; t < Tk; ++t) {
                 float bv = -INFINITY;
                 int bp = 0x7fffffff;
-                for (int e = lane; e < nk; e += kWave) {
-                    const float kv = kp[e];
-                    const bool after = kv < pv || (kv == pv && e > pp);
+                for (int e0 = 0; e0 < nk; e0 += kWave) {
+                    const int e = e0 + lane;
+                    const float kv = e < nk ? kp[e] : 0.0f;
+                    const bool after = e < nk && (kv < pv || (kv == pv && e > pp));
                     if (after && (kv > bv || (kv == bv && e < bp))) {
                         bv = kv;
                         bp = e;
@@ -2938,11 +2953,11 @@ __global__ __launch_bounds__(kWave) void euclid_refine_select_kernel(StageArgs a
                         bp = op;
                     }
                 }
-                pv = bv;
-                pp = bp;
+                pv = wave_uniform(bv);
+                pp = __builtin_amdgcn_readfirstlane(bp);
             }
             vT = pv;
-            ok = __builtin_amdgcn_readfirstlane(vT - vT == 0.0f ? 1 : 0) != 0;
+            ok = vT - vT == 0.0f;
         }
         if (ok) {
             const float thr = vT - 2.0f * E;
@@ -2969,7 +2984,7 @@ __global__ __launch_bounds__(kWave) void euclid_refine_select_kernel(StageArgs a
             if (RECIPE == HIGGS && lane == 0) x2s = sum_squares_k<K>(xs);
         }
         __syncthreads();
-        const float x2c = RECIPE == HIGGS ? x2s : 0.0f;
+        const float x2c = RECIPE == HIGGS ? wave_uniform(x2s) : 0.0f;
         if (ok) exact_values_frame<RECIPE, Q8, K>(a, xs, x2c, xq, xd, cand_n, cand_v, ncand, lane);
         __syncthreads();
 
@@ -2985,8 +3000,8 @@ __global__ __launch_bounds__(kWave) void euclid_refine_select_kernel(StageArgs a
         int win = 0;
         if (ok) {
             for (int c = 0; c < ncand; ++c) {
-                float cv = cand_v[c];
-                int cn = cand_n[c];
+                float cv = wave_uniform(cand_v[c]);
+                int cn = __builtin_amdgcn_readfirstlane(cand_n[c]);
 #pragma unroll
                 for (int r = 0; r < 5; ++r) {
                     const bool before = a.topk == 0 ? ranks_before<RECIPE>(cv, cn, sel_v[r], sel_n[r])

@@ -1440,12 +1440,14 @@ __device__ int select_group(const StageArgs &a, int64_t m_base, const float (&to
         constexpr int P = K <= 256 ? 4 : (K <= 512 ? 2 : 1);
         const int j = lane & 7, grp = lane >> 3;
         const int jw = q8_lane_word(j);
-        for (int e0 = grp; e0 < qcount; e0 += 8 * P) {
+        // a scalar trip count: the kernels that hold this loop spill
+        for (int b0 = 0; b0 < qcount; b0 += 8 * P) {
+            const int e0 = b0 + grp;
             int cq[P][K / 32], xw[P][K / 32], fs[P], n[P];
             float cd[P][K / 32], xd[P][K / 32], e2v[P], x2v[P];
 #pragma unroll
             for (int p = 0; p < P; ++p) {
-                const int e = e0 + 8 * p < qcount ? e0 + 8 * p : e0;
+                const int e = e0 + 8 * p < qcount ? e0 + 8 * p : qcount - 1;   // past the end: the last again, not written
                 fs[p] = q_f[e];
                 n[p] = q_n[e];
             }
@@ -3486,8 +3488,8 @@ __global__ __launch_bounds__(kNwThreads, 1) void euclid_narrow_kernel(CascadeArg
     const int N = c.a.N;
     const int64_t m_tile = static_cast<int64_t>(blockIdx.x) * LY::FRAMES;
     if (m_tile >= M) return;   // block-uniform
-    for (int i = threadIdx.x; i < LY::FRAMES; i += kNwThreads)
-        if (m_tile + i < M) c.bad_stage[m_tile + i] = c.a.Q;
+    static_assert(LY::FRAMES <= kNwThreads && LY::FRAMES * (K / 4) % kNwThreads == 0, "whole passes of the block");
+    if (threadIdx.x < LY::FRAMES && m_tile + threadIdx.x < M) c.bad_stage[m_tile + threadIdx.x] = c.a.Q;
 
     int lbits = 0;   // bits of the lane-local code index (N/4 codes per lane)
     while ((1 << lbits) < N / 4) ++lbits;
@@ -3498,8 +3500,9 @@ __global__ __launch_bounds__(kNwThreads, 1) void euclid_narrow_kernel(CascadeArg
     const int nb = wave < nblk ? (nblk - wave + kNwWaves - 1) / kNwWaves : 0;   // this wave's 16-code blocks
 
     // the stage-0 input (rows past M read row M - 1)
-    for (int e = threadIdx.x; e < LY::FRAMES * (K / 4); e += kNwThreads) {
-        const int f = e / (K / 4), k = e % (K / 4) * 4;
+#pragma unroll 1
+    for (int e0 = 0; e0 < LY::FRAMES * (K / 4); e0 += kNwThreads) {
+        const int e = e0 + threadIdx.x, f = e / (K / 4), k = e % (K / 4) * 4;
         const int64_t m = m_tile + f < M ? m_tile + f : M - 1;
         *reinterpret_cast<f32x4 *>(xr + f * LY::XSTR + k) = *reinterpret_cast<const f32x4 *>(c.x0 + m * K + k);
     }
@@ -3715,8 +3718,9 @@ __global__ __launch_bounds__(kNwThreads, 1) void euclid_narrow_kernel(CascadeArg
     // the residual after the last stage
     if (c.write_last) {
         __syncthreads();
-        for (int e = threadIdx.x; e < LY::FRAMES * (K / 4); e += kNwThreads) {
-            const int f = e / (K / 4), k = e % (K / 4) * 4;
+#pragma unroll 1
+        for (int e0 = 0; e0 < LY::FRAMES * (K / 4); e0 += kNwThreads) {
+            const int e = e0 + threadIdx.x, f = e / (K / 4), k = e % (K / 4) * 4;
             if (m_tile + f < M)
                 *reinterpret_cast<f32x4 *>(c.work + (m_tile + f) * K + k) = *reinterpret_cast<const f32x4 *>(xr + f * LY::XSTR + k);
         }

@@ -39,9 +39,12 @@ static_assert(kPcThreads == kScanThreads, "the exact scan's selection takes the 
 // many (a remainder's conditional steps made the compiler copy the ring every
 // round, waiting for all of it).
 constexpr int kAhead = 4;
-// Loops of these kernels run through scalar conditions (whole waves), not the
-// execution mask: where a kernel spills, ROCm 7.2's compiler has put spill
-// stores and reloads behind such a loop's exit, where no lane is active.
+// Loops of these kernels, select_group's among them, run through scalar
+// conditions (whole waves), not the execution mask: where a kernel spills,
+// ROCm 7.2's compiler has put spill stores and reloads behind such a loop's
+// exit, where no lane is active.  (All variants but the F32 ones of four
+// frames spill, up to 78 registers; tests/test_kernel_code.py holds the count
+// and looks at the built code.)
 // Widest hidden size: rows are this far apart, so that a frame's offset is an
 // immediate (as a run-time stride the addresses of F rows cost the registers
 // of the chains).
@@ -80,10 +83,12 @@ struct PcLayout {
     }
 };
 
-// The projection phases are calls of their own: inlined, their registers and
-// the search's add up and spill.  LDS goes to them as LDS pointers (a generic
-// pointer would make every read a flat one), what is uniform back into
-// scalar registers.
+// The Q8_0 projection phases and the exact scan are calls of their own:
+// inlined, their registers and the search's add up and spill.  project_f32 is
+// inlined: as a call it left its kernels of 4 and 8 frames with 4 and 40
+// spilled registers, for 0 and 18.  LDS goes to the projections as LDS
+// pointers (a generic pointer would make every read a flat one), what is
+// uniform back into scalar registers.
 typedef __attribute__((address_space(3))) float lds_float;
 typedef __attribute__((address_space(3))) int lds_int;
 typedef __attribute__((address_space(3))) f32x4 lds_f32x4;

@@ -1184,53 +1184,64 @@ __global__ __launch_bounds__(256) void dac_any_kernel(DacAnyArgs a) {
 using EncodeFn = void (*)(const float *, int64_t, int, int, const float4 *, int64_t, int64_t, const float *, int32_t *,
                           float *, float *, const int32_t *, int32_t *, int, int, float, int, float, int64_t, int, int);
 
-constexpr int kPrefetch = 12;   // float4 per thread in the prefetching variant
-// ... and of waves with one frame, whose registers have room (not with the
-// recon rows and the tinyBLAS order's): blocks of 4 waves hold the next image
-// of D = N = 1 024 too.  Eight stages of 647 frames 61 us without, 29 with.
-// A codebook in memory has the smaller prefix to hold: 17 pieces' clamped
-// loads cost its single stage 13 us.
-constexpr int prefetch_of(int fw, bool recon, int order) { return fw == 1 && !(recon && order == 1) ? 17 : kPrefetch; }
+// float4 pieces of the next stage's image that a thread holds: 12, or 17 for
+// waves with one frame, whose registers have room (not with the recon rows
+// and the tinyBLAS order's), where the image needs them: blocks of 4 waves
+// hold D = N = 1 024 too.  Eight stages of 647 frames 61 us without, 29 with.
+// Pieces past the image are clamped loads of its last one: where 12 hold it,
+// 17 cost time (9 needed, blocks of 8 waves, 1 100 frames of 9 stages: 41.8 us
+// with 17, 38.3 with 12; a single stage with its codebook in memory 13 us).
+// 0: the image is not held.
+constexpr int kPrefetch = 12, kPrefetchWide = 17;
+constexpr bool holds_wide(int fw, bool recon, int order) { return fw == 1 && !(recon && order == 1); }
+int held_pieces(int64_t img_f4, int threads, int fw, bool recon, int order, bool cbg) {
+    const int64_t need = (img_f4 + threads - 1) / threads;
+    if (need <= kPrefetch) return kPrefetch;
+    return need <= kPrefetchWide && !cbg && holds_wide(fw, recon, order) ? kPrefetchWide : 0;
+}
 
 // Variants: image copied at each stage start, prefetched a stage ahead, or
 // (large codebooks) the W_in + b_in prefix prefetched with c_hat in memory.
 // ORDER: the in-projection's summation order, 0 ggml_vec_dot_f32, 1 tinyBLAS.
 template <int DI, int FW, bool RECON, int ORDER>
-EncodeFn pick_pf(bool prefetch, bool cbg) {
+EncodeFn pick_pf(int held, bool cbg) {
     if (cbg) return dac_encode_kernel<DI, FW, RECON, kPrefetch, true, ORDER>;
-    return prefetch ? dac_encode_kernel<DI, FW, RECON, prefetch_of(FW, RECON, ORDER), false, ORDER>
-                    : dac_encode_kernel<DI, FW, RECON, 0, false, ORDER>;
+    if constexpr (holds_wide(FW, RECON, ORDER)) {
+        if (held == kPrefetchWide) return dac_encode_kernel<DI, FW, RECON, kPrefetchWide, false, ORDER>;
+    }
+    return held ? dac_encode_kernel<DI, FW, RECON, kPrefetch, false, ORDER>
+                : dac_encode_kernel<DI, FW, RECON, 0, false, ORDER>;
 }
 
 template <int DI, int FW, int ORDER>
-EncodeFn pick_recon(bool recon, bool prefetch, bool cbg) {
-    return recon ? pick_pf<DI, FW, true, ORDER>(prefetch, cbg) : pick_pf<DI, FW, false, ORDER>(prefetch, cbg);
+EncodeFn pick_recon(bool recon, int held, bool cbg) {
+    return recon ? pick_pf<DI, FW, true, ORDER>(held, cbg) : pick_pf<DI, FW, false, ORDER>(held, cbg);
 }
 
 template <int DI, int ORDER>
-EncodeFn pick_fw(int fw, bool recon, bool prefetch, bool cbg) {
+EncodeFn pick_fw(int fw, bool recon, int held, bool cbg) {
     switch (fw) {
-        case 1: return pick_recon<DI, 1, ORDER>(recon, prefetch, cbg);
-        case 2: return pick_recon<DI, 2, ORDER>(recon, prefetch, cbg);
-        default: return pick_recon<DI, 3, ORDER>(recon, prefetch, cbg);
+        case 1: return pick_recon<DI, 1, ORDER>(recon, held, cbg);
+        case 2: return pick_recon<DI, 2, ORDER>(recon, held, cbg);
+        default: return pick_recon<DI, 3, ORDER>(recon, held, cbg);
     }
 }
 
 template <int ORDER>
-EncodeFn pick_kernel_o(int64_t D, int fw, bool recon, bool prefetch, bool cbg) {
+EncodeFn pick_kernel_o(int64_t D, int fw, bool recon, int held, bool cbg) {
     switch (D / kWave) {
-        case 1: return pick_fw<1, ORDER>(fw, recon, prefetch, cbg);
-        case 2: return pick_fw<2, ORDER>(fw, recon, prefetch, cbg);
-        case 4: return pick_fw<4, ORDER>(fw, recon, prefetch, cbg);
-        case 8: return pick_fw<8, ORDER>(fw, recon, prefetch, cbg);
-        case 12: return pick_fw<12, ORDER>(fw, recon, prefetch, cbg);
-        case 16: return pick_fw<16, ORDER>(fw, recon, prefetch, cbg);
+        case 1: return pick_fw<1, ORDER>(fw, recon, held, cbg);
+        case 2: return pick_fw<2, ORDER>(fw, recon, held, cbg);
+        case 4: return pick_fw<4, ORDER>(fw, recon, held, cbg);
+        case 8: return pick_fw<8, ORDER>(fw, recon, held, cbg);
+        case 12: return pick_fw<12, ORDER>(fw, recon, held, cbg);
+        case 16: return pick_fw<16, ORDER>(fw, recon, held, cbg);
         default: return nullptr;
     }
 }
 
-EncodeFn pick_kernel(int64_t D, int fw, bool recon, bool prefetch, bool cbg, int order = 0) {
-    return order == 1 ? pick_kernel_o<1>(D, fw, recon, prefetch, cbg) : pick_kernel_o<0>(D, fw, recon, prefetch, cbg);
+EncodeFn pick_kernel(int64_t D, int fw, bool recon, int held, bool cbg, int order = 0) {
+    return order == 1 ? pick_kernel_o<1>(D, fw, recon, held, cbg) : pick_kernel_o<0>(D, fw, recon, held, cbg);
 }
 
 using MsFn = void (*)(const float *, int64_t, int, int, const float4 *, int64_t, const float *, int32_t *, float *,
@@ -1273,7 +1284,7 @@ MsFn pick_ms(int64_t D, bool recon, int order) {
 struct Shape {
     int fw = 1;
     int waves_per_block = 4;
-    bool prefetch = false;
+    int held = 0;   // float4 of the next stage's image per thread
 };
 
 Shape launch_shape(int64_t M, int64_t D, int64_t img_f4, bool recon, int num_cus, size_t lds_bytes, bool cbg,
@@ -1288,12 +1299,12 @@ Shape launch_shape(int64_t M, int64_t D, int64_t img_f4, bool recon, int num_cus
         if (env_fw >= 1 && env_fw <= 3 && fw != env_fw) continue;
         for (int wpb : {4, 6, 8}) {
             if (env_wpb && wpb != env_wpb) continue;
-            bool prefetch = (img_f4 + wpb * kWave - 1) / (wpb * kWave) <= (cbg ? kPrefetch : prefetch_of(fw, recon, order));
-            if (const char *e = std::getenv("AQ_DAC_PF")) prefetch = prefetch && std::atoi(e) != 0;
-            if (cbg && !prefetch) continue;   // the in-memory codebook variant always prefetches
+            int held = held_pieces(img_f4, wpb * kWave, fw, recon, order, cbg);
+            if (const char *e = std::getenv("AQ_DAC_PF")) held = std::atoi(e) != 0 ? held : 0;
+            if (cbg && !held) continue;   // the in-memory codebook variant always prefetches
             hipFuncAttributes attr{};
             int64_t simd_waves = 8;
-            const void *kfn = reinterpret_cast<const void *>(pick_kernel(D, fw, recon, prefetch, cbg, order));
+            const void *kfn = reinterpret_cast<const void *>(pick_kernel(D, fw, recon, held, cbg, order));
             if (hipFuncGetAttributes(&attr, kfn) == hipSuccess && attr.numRegs > 0)
                 simd_waves = std::min<int64_t>(8, 512 / ((attr.numRegs + 7) / 8 * 8));
             // The block must fit on a CU at all (waves per SIMD by registers,
@@ -1304,16 +1315,16 @@ Shape launch_shape(int64_t M, int64_t D, int64_t img_f4, bool recon, int num_cus
             const int64_t waves = (M + fw - 1) / fw;
             const int64_t blocks = (waves + wpb - 1) / wpb;
             const int64_t per_simd = ((blocks + cus - 1) / cus) * ((wpb * fw + 3) / 4);
-            const int64_t rank = per_simd * 64 + (prefetch ? 0 : 16) + (wpb == 8 ? 0 : 8) + (3 - fw);
+            const int64_t rank = per_simd * 64 + (held ? 0 : 16) + (wpb == 8 ? 0 : 8) + (3 - fw);
             if (std::getenv("AQ_DEBUG"))
                 std::fprintf(stderr, "aq_dac shape fw=%d wpb=%d pf=%d regs=%d blocks=%lld per_simd=%lld rank=%lld\n", fw,
-                             wpb, prefetch ? 1 : 0, attr.numRegs, (long long)blocks, (long long)per_simd,
+                             wpb, held, attr.numRegs, (long long)blocks, (long long)per_simd,
                              (long long)rank);
             if (rank < best_rank) {
                 best_rank = rank;
                 best.fw = fw;
                 best.waves_per_block = wpb;
-                best.prefetch = prefetch;
+                best.held = held;
             }
         }
     }
@@ -1586,13 +1597,13 @@ aq_status aq_dac_upload_ex(aq_ctx *ctx, int64_t Q, int64_t D, int64_t N, const f
     // The fused kernel's shapes: D a multiple of 64 with a register tile
     // (64 ... 1024), N a multiple of 64 up to 2^20; anything else takes the
     // any-shape kernel.
-    if (D % kWave != 0 || N % kWave != 0 || N > (int64_t{1} << 20) || !pick_kernel(D, 1, false, false, false))
+    if (D % kWave != 0 || N % kWave != 0 || N > (int64_t{1} << 20) || !pick_kernel(D, 1, false, 0, false))
         return upload_any(ctx, Q, D, N, w_in, b_in, codebook, w_out, b_out, recipe, out);
     int64_t img = image_f4(D, N);
     // c_hat read from memory when the whole stage image does not fit in LDS
     // next to the kernel's static LDS
     const bool cbg = static_cast<size_t>(img) * 16 >
-                     aq_lds_budget(reinterpret_cast<const void *>(pick_kernel(D, 1, false, false, false)));
+                     aq_lds_budget(reinterpret_cast<const void *>(pick_kernel(D, 1, false, 0, false)));
     aq_device_guard g(ctx->device);
 
     aq_dac_stages *st = new (std::nothrow) aq_dac_stages();
@@ -1834,7 +1845,7 @@ aq_status aq_dac_encode_ex(aq_ctx *ctx, const aq_dac_stages *st, const float *x,
             return dac_check_forced(ctx, st, force_idx);
         }
     }
-    EncodeFn fn = pick_kernel(st->D, fw, recon != nullptr, shape.prefetch, st->cbg, order);
+    EncodeFn fn = pick_kernel(st->D, fw, recon != nullptr, shape.held, st->cbg, order);
     const size_t rt_bytes = order == 1 ? static_cast<size_t>(shape.waves_per_block) * static_cast<size_t>(st->D) * 4 : 0;
     // A second stage image in LDS when it fits: one barrier per stage.
     const size_t budget = aq_lds_budget(reinterpret_cast<const void *>(fn));

@@ -1,8 +1,10 @@
-"""GPU parity of the DAC cascade at batches of one frame per wave: 4-wave
-blocks whose threads hold the next stage's image (D = N = 1 024: the last
-piece is a partial one), codebook chunks that are no multiple of the unrolled
+"""GPU parity of the DAC cascade at batches of one frame per wave: blocks of
+4, 6 and 8 waves whose threads hold the next stage's image (D = N = 1 024:
+17 pieces at 4 waves, the last a partial one, 12 at more), codebook chunks that are no multiple of the unrolled
 step, a codebook read from memory, both summation orders, with and without
 the reconstruction; channel-major input with ragged tiles; bit for bit."""
+
+import re
 
 import numpy as np
 import pytest
@@ -12,6 +14,7 @@ from test_dac_gpu import _sha
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("wpb", [4, 6, 8])
 @pytest.mark.parametrize("T,D,N,channel_major,recon", [
     (1, 1024, 1024, False, False),
     (647, 1024, 1024, True, False),    # 162 blocks of 4 waves; the gather's last tile of 7 frames
@@ -21,7 +24,7 @@ pytestmark = pytest.mark.gpu
     (5, 1024, 4096, False, False),     # codebook in memory
     (63, 256, 64, True, True),
 ])
-def test_dac_one_frame_per_wave(monkeypatch, T, D, N, channel_major, recon):
+def test_dac_one_frame_per_wave(monkeypatch, T, D, N, channel_major, recon, wpb):
     import torch
 
     if not torch.cuda.is_available():
@@ -30,9 +33,9 @@ def test_dac_one_frame_per_wave(monkeypatch, T, D, N, channel_major, recon):
     from aqmi import synth
     from oracle import Oracle
 
-    print(f"[gpu] dac one frame per wave T={T} D={D} N={N} cm={channel_major} recon={recon}", flush=True)
+    print(f"[gpu] dac one frame per wave T={T} D={D} N={N} cm={channel_major} recon={recon} waves={wpb}", flush=True)
     monkeypatch.setenv("AQ_DAC_FW", "1")
-    monkeypatch.setenv("AQ_DAC_WPB", "4")
+    monkeypatch.setenv("AQ_DAC_WPB", str(wpb))
     Q = 3
     cfg = dict(synth.dac_weights(91, Q, D, N, bias=True), x=synth.normal(91, 1, (T, D)), M=T, T=T, B=1, D=D, N=N, Q=Q)
     st = aqmi.DacStages(aqmi.Context(0), cfg["w_in"], cfg.get("b_in"), cfg["codebook"], cfg["w_out"], cfg.get("b_out"))
@@ -46,6 +49,39 @@ def test_dac_one_frame_per_wave(monkeypatch, T, D, N, channel_major, recon):
     ref = Oracle().dac_rvq(cfg)
     assert np.array_equal(idx.cpu().numpy(), ref["idx"])
     assert _sha(res.cpu().numpy()) == _sha(ref["residual"])
+    if recon:
+        assert _sha(rec.cpu().numpy()) == _sha(ref["recon"])
+
+
+@pytest.mark.parametrize("recon", [False, True])
+def test_dac_held_pieces_follow_the_block(monkeypatch, capfd, recon):
+    """Blocks that need no more than 12 pieces hold 12, whatever the frames per
+    wave; wider blocks of one frame per wave hold 17 (tinyBLAS order with
+    recon: the image is copied)."""
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import aqmi
+    from aqmi import synth
+    from oracle import Oracle
+
+    T, D, N, Q = 1100, 1024, 1024, 2   # a multiple of 4: the tinyBLAS order
+    cfg = dict(synth.dac_weights(91, Q, D, N, bias=True), x=synth.normal(91, 1, (T, D)), M=T, T=T, B=1, D=D, N=N, Q=Q)
+    st = aqmi.DacStages(aqmi.Context(0), cfg["w_in"], cfg.get("b_in"), cfg["codebook"], cfg["w_out"], cfg.get("b_out"))
+    x = torch.from_numpy(cfg["x"]).cuda()
+    idx = torch.full((T, Q), -1, dtype=torch.int32, device="cuda")
+    rec = torch.empty((T, D), dtype=torch.float32, device="cuda") if recon else None
+    capfd.readouterr()
+    monkeypatch.setenv("AQ_DEBUG", "1")
+    st.encode(x, T, idx, None, rec)
+    torch.cuda.synchronize()
+    held = {(int(fw), int(wpb)): int(pf) for fw, wpb, pf in
+            re.findall(r"shape fw=(\d) wpb=(\d) pf=(\d+)", capfd.readouterr().err)}
+    assert held[1, 4] == (0 if recon else 17)
+    assert held[1, 6] == held[1, 8] == held[2, 8] == 12
+    ref = Oracle().dac_rvq(cfg)
+    assert np.array_equal(idx.cpu().numpy(), ref["idx"])
     if recon:
         assert _sha(rec.cpu().numpy()) == _sha(ref["recon"])
 

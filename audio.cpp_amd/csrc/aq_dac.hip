@@ -955,6 +955,7 @@ __global__ void dac_table_kernel(const float *__restrict__ cb, const float *__re
 // recon[m][d] = sum over stages of z[s][idx[m][s]][d] (decode recipe).
 // (accumulate: out already holds the sum of earlier stages, which the z of
 // these stages are added to in order.)
+template <int B>
 __global__ void dac_decode_kernel(const int32_t *__restrict__ idx, int64_t ld, int64_t M, int Q, int64_t N, int64_t D,
                                   const float *__restrict__ tables, float *__restrict__ out,
                                   int32_t *__restrict__ flags, int accumulate) {
@@ -963,10 +964,9 @@ __global__ void dac_decode_kernel(const int32_t *__restrict__ idx, int64_t ld, i
     const int64_t m = t / D;
     const int64_t d = t % D;
     float acc = accumulate ? out[t] : 0.0f;
-    // Eight stages' codes, then their rows, at once (past the last stage: the
+    // B stages' codes, then their rows, at once (past the last stage: the
     // last again, not added): one by one, each stage waited for its code and
     // then for its row (1 291 frames of 8 stages: 12.3 us).
-    constexpr int B = 8;
     for (int s0 = 0; s0 < Q; s0 += B) {
         int32_t code[B];
         float z[B];
@@ -1883,7 +1883,12 @@ aq_status aq_dac_decode_ex(aq_ctx *ctx, const aq_dac_stages *st, const int32_t *
     aq_device_guard g(ctx->device);
     AQ_HIP(ctx, hipMemsetAsync(ctx->d_flags, 0, sizeof(int32_t) * AQ_FLAG_COUNT, ctx->stream));
     const int64_t total = M * st->D;
-    hipLaunchKernelGGL(dac_decode_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, ctx->stream, idx,
+    // as many stages at once as there are, up to eight: 40 000 frames of one
+    // stage 100 us, 196 with eight at once, which load its row eight times;
+    // of two 114 and 197, of four 145 and 199
+    const auto decode = st->Q == 1 ? dac_decode_kernel<1> : st->Q == 2 ? dac_decode_kernel<2>
+                        : st->Q <= 4 ? dac_decode_kernel<4> : dac_decode_kernel<8>;
+    hipLaunchKernelGGL(decode, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, ctx->stream, idx,
                        idx_ld, M, static_cast<int>(st->Q), st->N, st->D, st->d_tables, out, ctx->d_flags,
                        accumulate ? 1 : 0);
     AQ_HIP(ctx, hipGetLastError());

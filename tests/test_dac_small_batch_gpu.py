@@ -103,3 +103,36 @@ def test_outetts_waves_per_block(M):
     want = Oracle().outetts_rvq(cfg)
     assert np.array_equal(got["idx"], want["idx"])
     assert _sha(got["residual"]) == _sha(want["residual"])
+
+
+@pytest.mark.parametrize("Q", [1, 2, 3, 5, 8, 9, 17])   # one, two, four and eight stages' rows at once, with remainders
+def test_dac_decode_stage_counts(Q):
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import aqmi
+    from aqmi import synth
+    from oracle import Oracle
+
+    print(f"[gpu] dac decode Q={Q}", flush=True)
+    T, D, N = 37, 128, 64
+    cfg = dict(synth.dac_weights(93, Q, D, N, bias=True), x=synth.normal(93, 1, (T, D)), M=T, T=T, B=1, D=D, N=N, Q=Q)
+    st = aqmi.DacStages(aqmi.Context(0), cfg["w_in"], cfg.get("b_in"), cfg["codebook"], cfg["w_out"], cfg.get("b_out"))
+    codes = np.random.default_rng(3).integers(0, N, (T, Q)).astype(np.int32)
+    recon = Oracle().dac_rvq(cfg, codes)["recon"]   # teacher forced: the sum over these codes
+    idx = torch.from_numpy(codes).cuda()
+    out = torch.empty((T, D), dtype=torch.float32, device="cuda")
+    st.decode(idx, out)
+    assert _sha(out.cpu().numpy()) == _sha(recon)
+    first = torch.from_numpy(synth.normal(93, 2, (T, D))).cuda()   # one stage added to what is there
+    one = aqmi.DacStages(aqmi.Context(0), *(cfg[k][:1] for k in ("w_in", "b_in", "codebook", "w_out", "b_out")))
+    z0 = torch.empty_like(out)
+    one.decode(idx[:, :1].contiguous(), z0)
+    want = first + z0
+    one.decode_ex(idx.data_ptr(), Q, T, first, True)
+    assert _sha(first.cpu().numpy()) == _sha(want.cpu().numpy())
+    idx[T - 1, Q - 1] = N
+    with pytest.raises(aqmi.AqError) as e:
+        st.decode(idx, out)
+    assert e.value.status == 3

@@ -600,12 +600,14 @@ aq_status aq_outetts_launch(aq_ctx *ctx, const aq_outetts_args &args) {
     const size_t win = static_cast<size_t>(8) * (a.D + 4) * sizeof(float), chat = static_cast<size_t>(8) * a.N * sizeof(float);
     int nw = kOtW;
     while (nw > 1 && nw * per_wave + win > budget) --nw;
-    // Few frames: fewer waves, so that the blocks spread over the CUs, but two
-    // at least to stage the tables (1 046 frames: 2, 3, 4, 6 waves 47.9, 48.2,
-    // 51.0, 54.5 us, one 106).
+    // Few frames: fewer waves, so that the blocks spread over the CUs, but
+    // three at least to stage the tables: every block copies them, and a
+    // block of two waits longest for memory.  1 046 frames with 2, 3, 4, 6
+    // waves: 48.1, 48.3, 50.2, 54.8 us with the tables in L2, 78.5, 68.8, 69.0,
+    // 72.0 us with nothing in a cache.
     const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
     const int64_t spread = (a.M + kHF * cus - 1) / (kHF * cus);
-    nw = static_cast<int>(std::min<int64_t>(nw, std::max<int64_t>(2, spread)));
+    nw = static_cast<int>(std::min<int64_t>(nw, std::max<int64_t>(3, spread)));
     size_t lds = nw * per_wave;
     a.win_lds = lds + win <= budget ? 1 : 0;
     if (a.win_lds) lds += win;

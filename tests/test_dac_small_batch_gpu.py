@@ -86,7 +86,7 @@ def test_dac_held_pieces_follow_the_block(monkeypatch, capfd, recon):
         assert _sha(rec.cpu().numpy()) == _sha(ref["recon"])
 
 
-@pytest.mark.parametrize("M", [9, 2049, 5121])   # 2, 3 and 6 waves per block, the last one of one frame
+@pytest.mark.parametrize("M", [9, 2049, 4097, 5121])   # 3, 3, 5 and 6 waves per block, the last one of one frame
 def test_outetts_waves_per_block(M):
     import torch
 

@@ -288,7 +288,6 @@ aq_status euclid_alloc(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, bool q8, bo
     bool ok = hipMalloc(&cb->d_cbh, QNK * 2) == hipSuccess && hipMalloc(&cb->d_cbl, QNK * 2) == hipSuccess &&
               hipMalloc(&cb->d_hh, QN * 4) == hipSuccess && hipMalloc(&cb->d_cbf, QNK * 4) == hipSuccess &&
               hipMalloc(&cb->d_bias, QN * 4) == hipSuccess && hipMalloc(&cb->d_e2, QN * 4) == hipSuccess;
-    if (ok && !any && K == 256) ok = hipMalloc(&cb->d_cbx, QNK * 2) == hipSuccess;
     if (ok && q8) ok = hipMalloc(&cb->d_q8, QNK) == hipSuccess && hipMalloc(&cb->d_q8d, QNK / 32 * 4) == hipSuccess;
     if (!ok) {
         aq_euclid_release(cb);
@@ -357,12 +356,6 @@ aq_status euclid_prepare(aq_ctx *ctx, aq_codebooks *cb) {
         hipLaunchKernelGGL(euclid_prep_kernel, grid, block, 0, ctx->stream, cb->d_cbf, QN, cb->N,
                            static_cast<int>(cb->K), cb->d_cbh, cb->d_cbl, cb->d_hh, cb->d_bias, cb->d_e2, smax,
                            nonfinite);
-        if (cb->d_cbx) {
-            const int64_t pieces = QN * cb->K / 8;
-            hipLaunchKernelGGL(euclid_fragments_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
-                               ctx->stream, reinterpret_cast<const u32x4 *>(cb->d_cbh), pieces,
-                               static_cast<int>(cb->K), reinterpret_cast<u32x4 *>(cb->d_cbx));
-        }
         step = "launch";
         e = hipGetLastError();
         if (e == hipSuccess) {
@@ -413,8 +406,38 @@ aq_status euclid_prepare(aq_ctx *ctx, aq_codebooks *cb) {
     return st;
 }
 
+// Room for an image that only a faster path reads, or null: an upload whose
+// device memory ends here is not refused, its calls take the per-stage
+// launches (AQ_EUCLID_TEST_NO_IMAGE, a test hook, ends it).
+void *optional_image(size_t bytes) {
+    void *p = nullptr;
+    if (std::getenv("AQ_EUCLID_TEST_NO_IMAGE") || hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();   // not left for the next call to report
+        return nullptr;
+    }
+    return p;
+}
+
+// The codebook in fragment order, for the one-launch cascades.
+aq_status euclid_fragment_image(aq_ctx *ctx, aq_codebooks *cb) {
+    const int64_t pieces = cb->Q * cb->N * cb->K / 8;   // whole 16-code blocks: N is a multiple of the chunk
+    cb->d_cbx = static_cast<uint16_t *>(optional_image(static_cast<size_t>(pieces) * 16));
+    if (!cb->d_cbx) return AQ_OK;
+    hipLaunchKernelGGL(euclid_fragments_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
+                       ctx->stream, reinterpret_cast<const u32x4 *>(cb->d_cbh), pieces, static_cast<int>(cb->K),
+                       reinterpret_cast<u32x4 *>(cb->d_cbx));
+    AQ_HIP(ctx, hipGetLastError());
+    AQ_HIP(ctx, hipStreamSynchronize(ctx->stream));   // the handle may be used on another stream
+    return AQ_OK;
+}
+// ... where the narrow cascade reads it: plain codebooks of K = 256 (a
+// codebook that is not finite is scanned exactly).
+aq_status euclid_narrow_image(aq_ctx *ctx, aq_codebooks *cb) {
+    return cb->K == 256 && !cb->any && !cb->exact_only ? euclid_fragment_image(ctx, cb) : AQ_OK;
+}
+
 aq_status euclid_upload_from(aq_ctx *ctx, const char *fn, int64_t Q, int64_t N, int64_t K, int cb_type,
-                             const void *data, hipMemcpyKind kind, int recipe, aq_codebooks **out) {
+                             const void *data, hipMemcpyKind kind, int recipe, bool plain, aq_codebooks **out) {
     if (!ctx || !out || !data) return aq_fail(ctx, AQ_E_INVALID_ARG, "%s: null argument", fn);
     *out = nullptr;
     bool any = false;
@@ -425,6 +448,7 @@ aq_status euclid_upload_from(aq_ctx *ctx, const char *fn, int64_t Q, int64_t N, 
     st = euclid_alloc(ctx, Q, N, K, cb_type != AQ_CB_F32, any, recipe, &cb);
     if (st == AQ_OK) st = euclid_fill(ctx, cb, cb_type, data, kind);
     if (st == AQ_OK) st = euclid_prepare(ctx, cb);
+    if (st == AQ_OK && plain) st = euclid_narrow_image(ctx, cb);
     if (st != AQ_OK) {
         if (cb) aq_euclid_release(cb);
         return st;
@@ -439,13 +463,13 @@ extern "C" {
 
 aq_status aq_euclid_upload(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, int cb_type, const void *data, int recipe,
                            aq_codebooks **out) {
-    return euclid_upload_from(ctx, "aq_euclid_upload", Q, N, K, cb_type, data, hipMemcpyHostToDevice, recipe, out);
+    return euclid_upload_from(ctx, "aq_euclid_upload", Q, N, K, cb_type, data, hipMemcpyHostToDevice, recipe, true, out);
 }
 
 aq_status aq_euclid_upload_device(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, int cb_type, const void *data,
                                   int recipe, aq_codebooks **out) {
     return euclid_upload_from(ctx, "aq_euclid_upload_device", Q, N, K, cb_type, data, hipMemcpyDeviceToDevice, recipe,
-                              out);
+                              true, out);
 }
 
 aq_status aq_ema_codebook(aq_ctx *ctx, const float *embedding_sum, const float *cluster_usage, int64_t Q, int64_t N,
@@ -486,6 +510,7 @@ aq_status aq_euclid_upload_ema(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, con
         st = aq_fail(ctx, AQ_E_DEVICE, "aq_euclid_upload_ema: host to device copy failed");
     if (st == AQ_OK) st = aq_ema_codebook(ctx, d, d + QNK, Q, N, K, eps, cb->d_cbf);
     if (st == AQ_OK) st = euclid_prepare(ctx, cb);
+    if (st == AQ_OK) st = euclid_narrow_image(ctx, cb);
     (void)hipFree(d);
     if (st != AQ_OK) {
         aq_euclid_release(cb);
@@ -515,7 +540,8 @@ aq_status aq_euclid_upload_projected(aq_ctx *ctx, int64_t Q, int64_t N, int64_t 
         if (ls != AQ_OK) return ls;
     }
     aq_codebooks *cb = nullptr;
-    aq_status st = aq_euclid_upload(ctx, Q, N, K, cb_type, codebook, recipe, &cb);
+    aq_status st = euclid_upload_from(ctx, "aq_euclid_upload", Q, N, K, cb_type, codebook, hipMemcpyHostToDevice, recipe,
+                                      false, &cb);
     if (st != AQ_OK) return st;
     if (cb->any) {
         aq_euclid_release(cb);
@@ -525,18 +551,11 @@ aq_status aq_euclid_upload_projected(aq_ctx *ctx, int64_t Q, int64_t N, int64_t 
     }
     aq_device_guard g(ctx->device);
     st = aq_proj_create(ctx, Q, N, K, H, cb->d_cbf, proj_type, w_in, b_in, w_out, b_out, &cb->proj);
-    if (st == AQ_OK) st = aq_proj_cascade_weights(ctx, cb->proj);
-    if (st == AQ_OK && cb->proj->w_cx && !cb->d_cbx) {   // the cascade's codebook image
-        const int64_t pieces = Q * N * K / 8;
-        if (hipMalloc(&cb->d_cbx, static_cast<size_t>(pieces) * 16) != hipSuccess) {
-            st = aq_fail(ctx, AQ_E_NOMEM, "aq_euclid_upload: device allocation failed");
-        } else {
-            hipLaunchKernelGGL(euclid_fragments_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
-                               ctx->stream, reinterpret_cast<const u32x4 *>(cb->d_cbh), pieces, static_cast<int>(K),
-                               reinterpret_cast<u32x4 *>(cb->d_cbx));
-            if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess)
-                st = aq_fail(ctx, AQ_E_DEVICE, "aq_euclid_upload_projected: codebook image failed");
-        }
+    // the one-launch cascade's images, for shapes that it takes
+    if (st == AQ_OK && aq_proj_cascade_shape(cb->proj, N)) {
+        cb->proj->w_cx = optional_image(aq_proj_cascade_bytes(cb->proj));
+        if (cb->proj->w_cx) st = aq_proj_cascade_weights(ctx, cb->proj);
+        if (st == AQ_OK && cb->proj->w_cx) st = euclid_fragment_image(ctx, cb);
     }
     if (st != AQ_OK) {
         aq_euclid_release(cb);
@@ -958,7 +977,7 @@ aq_status euclid_encode_impl(aq_ctx *ctx, const aq_codebooks *cb, const aq_frame
     // fixed region keep the per-stage launches and their limits;
     // AQ_EUCLID_PIPELINE=stages asks for them too (comparisons and tests).
     const char *pipe_env = std::getenv("AQ_EUCLID_PIPELINE");
-    if (pw && !arena.base && cb->d_cbx && aq_proj_cascade_shape(pw, cb->N, M) &&
+    if (pw && pw->w_cx && cb->d_cbx && !arena.base && M >= 2 &&
         !(pipe_env && std::strcmp(pipe_env, "stages") == 0))
         return euclid_encode_projected(ctx, cb, in, M, idx, residual, dist, topk, topk_idx, topk_dist, force_idx, arena, topl);
     StageFn sweep = kk->sweep[cb->q8 ? 1 : 0][topl - 3];

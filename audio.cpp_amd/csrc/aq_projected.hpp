@@ -73,12 +73,14 @@ aq_status aq_proj_decode(aq_ctx *ctx, const aq_proj_weights *pw, const int32_t *
 aq_status aq_proj_check_lds(aq_ctx *ctx, int64_t H, bool q8, const char *fn);
 
 // The one-launch projected cascade (aq_projected_cascade.hip): whether its
-// kernels take the shape, its weight images (at upload), and the encode of
+// kernels take the shape (batches of two frames or more), its weight image's
+// size and contents (w_cx, at upload), and the encode of
 // c's frames through every stage (c: stage 0's codebook pointers, bounds,
 // counts and outputs; force: the update's codes or null; rout [M, H] or
 // null).
 namespace aq_euclid { struct CascadeArgs; }
-bool aq_proj_cascade_shape(const aq_proj_weights *pw, int64_t N, int64_t M);
+bool aq_proj_cascade_shape(const aq_proj_weights *pw, int64_t N);
+size_t aq_proj_cascade_bytes(const aq_proj_weights *pw);
 aq_status aq_proj_cascade_weights(aq_ctx *ctx, aq_proj_weights *pw);
 aq_status aq_proj_cascade(aq_ctx *ctx, const aq_proj_weights *pw, const aq_euclid::CascadeArgs &c, bool q8c, int recipe,
                           int topl, const aq_frames_desc &in, const int32_t *force, float *rout, bool timed);

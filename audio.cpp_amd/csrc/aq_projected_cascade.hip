@@ -803,16 +803,17 @@ int proj_frames(int64_t M, int cus) {
 
 }  // namespace
 
-bool aq_proj_cascade_shape(const aq_proj_weights *pw, int64_t N, int64_t M) {
-    return pw->K == kPcK && M >= 2 && N % 16 == 0 && N >= 64 && N <= kScanChunk && pw->w_cx != nullptr;
+bool aq_proj_cascade_shape(const aq_proj_weights *pw, int64_t N) {
+    return pw->K == kPcK && pw->H <= kPcH && pw->H % ((pw->q8 ? 128 : 64) * kAhead) == 0 && N % 16 == 0 && N >= 64 &&
+           N <= kScanChunk;
+}
+
+size_t aq_proj_cascade_bytes(const aq_proj_weights *pw) {
+    return static_cast<size_t>(pw->Q * pw->K * pw->H) * (pw->q8 ? 1 : 4);
 }
 
 aq_status aq_proj_cascade_weights(aq_ctx *ctx, aq_proj_weights *pw) {
-    if (pw->K != kPcK || pw->H > kPcH || pw->H % (pw->q8 ? 128 * kAhead : 64 * kAhead) != 0) return AQ_OK;
-    const int64_t QKH = pw->Q * pw->K * pw->H;
-    const int64_t n = pw->q8 ? QKH / 4 : QKH;   // dwords
-    if (hipMalloc(&pw->w_cx, static_cast<size_t>(n) * 4) != hipSuccess)
-        return aq_fail(ctx, AQ_E_NOMEM, "aq_euclid_upload_projected: device allocation or copy failed");
+    const int64_t n = static_cast<int64_t>(aq_proj_cascade_bytes(pw)) / 4;   // dwords
     const dim3 grid(static_cast<unsigned>((n + 255) / 256)), block(256);
     if (pw->q8)
         hipLaunchKernelGGL(pc_weights_q8_kernel, grid, block, 0, ctx->stream, reinterpret_cast<const int *>(pw->w_in_q), n,

@@ -1058,6 +1058,9 @@ aq_status euclid_encode_impl(aq_ctx *ctx, const aq_codebooks *cb, const aq_frame
             tile2 = tiles8;
         }
     }
+    if (std::getenv("AQ_DEBUG"))
+        std::fprintf(stderr, "aq_euclid sweep tiles=%lld splits=%d,%d from tile %lld\n", (long long)tiles, nsplit, nsplit2,
+                     (long long)tile2);
     const int maxsplit = nsplit2 > nsplit ? nsplit2 : nsplit;
     const int64_t sweep_blocks = tile2 * nsplit + (tiles8 - tile2) * nsplit2;
     const int64_t ngroups = (M + 15) / 16;

@@ -24,14 +24,14 @@ def torch():
     return t
 
 
-@pytest.fixture(autouse=True, params=["resident", "cascade", "stages"])
+@pytest.fixture(autouse=True, params=["default", "cascade", "stages"])
 def pipeline(request, monkeypatch):
-    """Every test runs on each encode pipeline: the default (the one-launch
-    cascade with the residual in registers for f32 codebooks at K = 256, the
-    per-stage kernels otherwise), the one-launch cascade with the residual in
+    """Every test runs on each encode pipeline: the default (the narrow
+    one-launch cascade, residual in LDS, at K = 256, the per-stage kernels
+    otherwise), the one-launch cascade with the residual in
     memory (AQ_EUCLID_PIPELINE=cascade) and the per-stage kernels
     (AQ_EUCLID_PIPELINE=stages)."""
-    if request.param == "resident":
+    if request.param == "default":
         monkeypatch.delenv("AQ_EUCLID_PIPELINE", raising=False)
     else:
         monkeypatch.setenv("AQ_EUCLID_PIPELINE", request.param)
@@ -40,7 +40,7 @@ def pipeline(request, monkeypatch):
 
 def effective(pipeline, K, cb_type=0):
     """The pipeline an encode takes under the `pipeline` fixture's setting."""
-    return "stages" if pipeline == "resident" and K != 256 else pipeline
+    return "stages" if pipeline == "default" and K != 256 else pipeline
 
 
 @pytest.fixture(scope="module")

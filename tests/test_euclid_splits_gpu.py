@@ -11,14 +11,14 @@ from test_euclid_gpu import bits, run
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M,K,N,recipe", [
-    (3, 512, 1024, "higgs"),        # 8 splits of 128 codes
-    (7, 768, 2048, "omnivoice"),    # 16
-    (33, 768, 4096, "higgs"),       # 32
-    (2, 512, 4096, "direct"),       # 32
-    (4097, 512, 1024, "higgs"),     # 33 tiles: past the rule, 4
+@pytest.mark.parametrize("M,K,N,recipe,splits", [
+    (3, 512, 1024, "higgs", 8),        # 128 codes a split
+    (7, 768, 2048, "omnivoice", 16),
+    (33, 768, 4096, "higgs", 32),
+    (2, 512, 4096, "direct", 32),
+    (4097, 512, 1024, "higgs", 4),     # 33 tiles: past the rule
 ])
-def test_split_counts(M, K, N, recipe):
+def test_split_counts(monkeypatch, capfd, M, K, N, recipe, splits):
     import torch
 
     if not torch.cuda.is_available():
@@ -28,12 +28,14 @@ def test_split_counts(M, K, N, recipe):
     from oracle import Oracle
 
     print(f"[gpu] splits M={M} K={K} N={N} {recipe}", flush=True)
+    monkeypatch.setenv("AQ_DEBUG", "1")
     cb = synth.normal(83, 1, (1, N, K))
     cb[0, N - 5] = cb[0, 5]   # equal codes, in the first and the last split
     x = synth.normal(83, 2, (M, K))
     x[0] = cb[0, 5]
     cfg = dict(x=x, M=M, K=K, Q=1, N=N, codebook=cb)
     out = run(torch, aqmi.Context(0), cb, getattr(aqmi, recipe.upper()), x)
+    assert f"splits={splits},{splits}" in capfd.readouterr().err
     oracle = Oracle()
     ref = {"omnivoice": oracle.euclid_rvq, "higgs": oracle.higgs_rvq, "direct": oracle.direct_rvq}[recipe](cfg)
     dist = -ref["logit"] if recipe == "omnivoice" else ref["dist"]

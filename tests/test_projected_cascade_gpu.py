@@ -97,3 +97,27 @@ def test_projected_cascade_block_edges(torch, ctx, oracle, monkeypatch, F, M, re
         assert np.array_equal(bits(a[~np.isnan(a)]), bits(b[~np.isnan(b)]))
     if topk:
         check_topk(got, ref)
+
+
+@pytest.mark.parametrize("F", [4, 8, 12])
+@pytest.mark.parametrize("q8", [False, True])
+def test_projected_cascade_channel_major(torch, ctx, oracle, monkeypatch, F, q8):
+    """[B, C, T] input whose clips end inside the blocks (2 clips of 23 frames)."""
+    import aqmi
+    from aqmi import synth
+
+    print(f"[gpu] projected channel-major F={F} q8={q8}", flush=True)
+    monkeypatch.setenv("AQ_PROJ_FRAMES", str(F))
+    B, T, H, N, Q = 2, 23, 1024, 256, 2
+    cfg = synth.projected_config(B * T, aqmi.HIGGS, seed=73, H=H, N=N, Q=Q, cb_q8=q8, proj_q8=q8)
+    cbt = aqmi.CB_Q8_0 if q8 else aqmi.CB_F32
+    cb, w_in, w_out = (cfg[k + "_q8" if q8 else k] for k in ("codebook", "w_in", "w_out"))
+    cbs = aqmi.Codebooks.projected(ctx, cb, w_in, cfg["b_in"], w_out, cfg["b_out"], aqmi.HIGGS, cbt, cbt)
+    x = torch.from_numpy(np.ascontiguousarray(cfg["x"].reshape(B, T, H).transpose(0, 2, 1))).cuda()
+    idx = torch.full((B * T, Q), -1, dtype=torch.int32, device="cuda")
+    res = torch.empty((B * T, H), dtype=torch.float32, device="cuda")
+    cbs.encode_strided(x, B * T, T, H * T, 1, T, idx, res)
+    torch.cuda.synchronize()
+    ref = oracle.projected_rvq(cfg)
+    assert np.array_equal(idx.cpu().numpy(), ref["idx"])
+    assert np.array_equal(bits(res.cpu().numpy()), bits(ref["residual"]))

@@ -28,6 +28,17 @@ def torch():
     return t
 
 
+@pytest.fixture(autouse=True, params=["default", "stages"])
+def pipeline(request, monkeypatch):
+    """Every test runs on the default pipeline (one launch for projected
+    cascades of width 64 and plain codebooks of K = 256) and on the per-stage
+    launches, which other shapes and the fixed region take."""
+    if request.param == "default":
+        monkeypatch.delenv("AQ_EUCLID_PIPELINE", raising=False)
+    else:
+        monkeypatch.setenv("AQ_EUCLID_PIPELINE", request.param)
+
+
 @pytest.fixture(scope="module")
 def ctx(torch):
     import aqmi
@@ -133,7 +144,10 @@ def test_projected_matches_golden(torch, ctx, tag, kw, topk):
 @pytest.mark.parametrize("kw,M,topk", [
     (dict(recipe=1), 1, 0), (dict(recipe=0), 1, 0), (dict(recipe=1, cb_q8=True, proj_q8=True), 1, 2),
     (dict(recipe=1, proj_q8=True), 37, 0), (dict(recipe=1, cb_q8=True), 50, 3),
-    (dict(recipe=0, H=512, K=256, N=512, Q=3), 77, 0), (dict(recipe=1, H=768, K=64, N=256, Q=2), 2, 1)])
+    (dict(recipe=0, H=512, K=256, N=512, Q=3), 77, 0), (dict(recipe=1, H=768, K=64, N=256, Q=2), 2, 1),
+    # hidden sizes that the one-launch cascade does not take
+    (dict(recipe=1, H=320, K=64, N=256, Q=2), 41, 0), (dict(recipe=1, H=768, K=64, N=256, Q=2, proj_q8=True), 37, 2),
+    (dict(recipe=0, H=1280, K=64, N=256, Q=2), 18, 0)])
 def test_projected_matches_oracle(torch, ctx, oracle, kw, M, topk):
     """Other weight types, one frame (ggml_vec_dot_f32 order), other widths
     and ragged M against the oracle."""

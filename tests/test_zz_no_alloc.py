@@ -76,13 +76,17 @@ def test_noalloc_q8_topk_matches_encode(torch, ctx):
     compare(torch, cbs, [x, x[:517].contiguous()], 4)
 
 
-def test_noalloc_projected_matches_encode(torch, ctx):
+@pytest.mark.parametrize("q8", [False, True])
+def test_noalloc_projected_matches_encode(torch, ctx, q8):
+    """(The fixed region's calls take the per-stage launches, encode's the
+    one-launch cascade.)"""
     import aqmi
     from aqmi import synth
 
-    cfg = synth.projected_config(300, recipe=1, Q=4)
-    cbs = aqmi.Codebooks.projected(ctx, cfg["codebook"], cfg["w_in"], cfg["b_in"], cfg["w_out"], cfg["b_out"],
-                                   aqmi.HIGGS)
+    cfg = synth.projected_config(300, recipe=1, Q=4, cb_q8=q8, proj_q8=q8)
+    cbt = aqmi.CB_Q8_0 if q8 else aqmi.CB_F32
+    cb, w_in, w_out = (cfg[k + "_q8" if q8 else k] for k in ("codebook", "w_in", "w_out"))
+    cbs = aqmi.Codebooks.projected(ctx, cb, w_in, cfg["b_in"], w_out, cfg["b_out"], aqmi.HIGGS, cbt, cbt)
     x = torch.from_numpy(cfg["x"]).cuda()
     compare(torch, cbs, [x, x[:64].contiguous()], 0)
 

@@ -226,7 +226,7 @@ struct aq_codebooks {
     bool any = false;
     uint16_t *d_cbh = nullptr;   // [Q][N][K] fp16(c)
     uint16_t *d_cbl = nullptr;   // [Q][N][K] fp16(c - fp16(c)) (refine pass)
-    uint16_t *d_cbx = nullptr;   // d_cbh in fragment order (K = 256: the narrow cascade)
+    uint16_t *d_cbx = nullptr;   // d_cbh in fragment order, for the one-launch cascades, or null
     float *d_hh = nullptr;       // [Q][N] -|c|^2 / 2 (fp32 of the double sum)
     float *d_cbf = nullptr;      // [Q][N][K]
     float *d_bias = nullptr;     // [Q][N] (OMNI)
@@ -734,10 +734,12 @@ aq_status euclid_encode_any(aq_ctx *ctx, const aq_codebooks *cb, const aq_frames
 // AQ_EUCLID_PIPELINE=stages asks for the per-stage pipeline and narrow1,
 // narrow2, narrow4 for the narrow cascade at that many frame groups.
 //
-// Frame groups per block: a round of blocks (one per CU) takes about 110, 120
-// and 157 us with one, two and four groups (8 stages of 2048 codes; the same
+// Frame groups per block: a round of blocks (one per CU) takes 107, 121 and
+// 162 us with one, two and four groups in a call of several rounds (48 000
+// frames, 8 stages of 2048 codes; 111, 125 and 171 us alone; the same
 // proportions for Q8_0 and DIRECT), so the count with the least rounds x time
-// runs: up to 16 frames per CU one group, up to 32 two, else mostly four.
+// (110, 120, 157) runs: up to 16 frames per CU one group, up to 32 two, else
+// mostly four.
 enum class Pipeline { kStages, kCascade, kNarrow };
 Pipeline pipeline_for(const aq_codebooks *cb, const KsKernels *kk, int var, int topl, int64_t M, int cus, int *fg) {
     if (cb->proj || cb->exact_only || !kk->cascade[var][topl - 3]) return Pipeline::kStages;

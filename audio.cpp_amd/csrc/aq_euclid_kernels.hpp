@@ -3417,12 +3417,17 @@ __global__ __launch_bounds__(kCThreads, 1) void euclid_cascade_kernel(CascadeArg
 // What bounds it: with one or two groups the codebook stream into the CU
 // (N K 2 bytes a stage, 42 bytes a cycle: 24 K of 31 K cycles a stage), with
 // four the MFMAs and key updates of two waves per SIMD (25 K of 38 K); then
-// the select's round trips.  Blocks share nothing, so the time is the same
-// for any number of blocks up to one per CU: 8 stages of 2048 codes took
-// 125 us for up to 4 096 frames (FG = 1), 129 us for 8 192 (FG = 2), 174 us
-// for 16 384 (FG = 4) and 471 us for 48 000.  The kernel it replaces (192
-// frames per block, each wave sweeping a whole codebook from LDS for its own
-// 48 frames, residual in AGPRs) took 434-502 us for any of these.
+// the select's round trips.  Blocks share nothing, so a round of one block
+// per CU takes about the same time for any number of them: 8 stages of 2048
+// codes 111 us for up to 4 096 frames (FG = 1), 125 us for 8 192 (FG = 2),
+// 137 to 171 us for up to 16 384 (FG = 4), 487 us for 48 000 (OmniVoice;
+// DIRECT 114, 128, 177, 504 us, Q8_0 115, 136, 176, 493 us).  Calls with the
+// kernel it replaces (192 frames per block, each wave sweeping a whole
+// codebook from LDS for its own 48 frames, residual in AGPRs) took 475 us for
+// 300 frames and 513 to 530 us for 48 000, with this one 122 and 482 to 507 on
+// the same boxes.  Small codebooks at whole rounds of that kernel (48 000
+// frames) are slower here: 64 codes 162 -> 172 us, 128 174 -> 181, 256 197 -> 198,
+// 512 241 -> 231.
 constexpr int kNwWaves = 8;
 constexpr int kNwThreads = kNwWaves * kWave;
 // A fragments in flight per wave (four frame groups leave room for one 16-code block)
@@ -3774,8 +3779,9 @@ __device__ inline bool same_bits(float x, float y) { return __float_as_uint(x) =
 // scan's); where the code differs from the cascade's, the frame's earliest
 // wrong stage is recorded for the fix-up, and where only the distance or
 // top-k list differ they are corrected in place.  F32 codebooks in tinyBLAS
-// order and Q8_0 codebooks take the values that euclid_verify_values_kernel
-// spread over the grid (up to a.scap pairs), or compute them in the block
+// order or under DIRECT and Q8_0 codebooks take the values that
+// euclid_verify_values_kernel spread over the grid (up to a.scap pairs), or
+// compute them in the block
 // (coalesced code-row reads: the quad layout, or 8 lanes per Q8_0 code).
 template <int RECIPE, bool Q8, int KS>
 __device__ inline void scan_frame(const StageArgs &a, const float *xs, const int8_t *xq, const float *xd, ScanSh &sh) {

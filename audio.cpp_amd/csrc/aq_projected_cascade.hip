@@ -22,7 +22,7 @@
 // cycle; Q8_0: four operations per 4-element dot), and for few frames the
 // weights' way into the CU (256 KB a stage).  The per-stage launches it
 // replaces (projection, sweep, select, refine pair, exact scan; 16 frames
-// per projection block) took 83 us a stage for 250 frames (now 11) and 177 us
+// per projection block) took 87 us a stage for 250 frames (now 11) and 177 us
 // for 6 000 frames with Q8_0 weights (now 44); more at proj_frames() below.
 #include "aq_euclid_kernels.hpp"
 #include "aq_projected.hpp"

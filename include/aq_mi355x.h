@@ -354,7 +354,9 @@ aq_status aq_euclid_upload_projected(aq_ctx *ctx, int64_t Q, int64_t N, int64_t 
  * took them or, when no more than 64 were open, the exact scan; in the
  * one-launch cascade (codebooks at K = 256) the frames that continued
  * with their best exactly evaluated candidate and were verified by the
- * exact scan afterwards (host int32 array; synchronises the stream).  A
+ * exact scan afterwards; in the one-launch projected cascade (width 64, two
+ * frames or more) the frames that their block scanned exactly (host int32
+ * array; synchronises the stream).  A
  * measurement aid with no reference counterpart. */
 aq_status aq_euclid_failures(aq_ctx *ctx, const aq_codebooks *cb, int32_t *host_counts);
 
@@ -362,7 +364,8 @@ aq_status aq_euclid_failures(aq_ctx *ctx, const aq_codebooks *cb, int32_t *host_
  * the exact scan decided: those the refine pass left open, or all open
  * frames when no more than 64 were; in the one-launch cascade the frames
  * whose verified continuation was wrong, recomputed from that stage on and
- * counted at each recomputed stage (host int32 array; synchronises the
+ * counted at each recomputed stage; in the one-launch projected cascade the
+ * same frames as aq_euclid_failures (host int32 array; synchronises the
  * stream).  A measurement aid with no reference counterpart. */
 aq_status aq_euclid_exact_scans(aq_ctx *ctx, const aq_codebooks *cb, int32_t *host_counts);
 

@@ -272,8 +272,33 @@ aq_status check_upload(aq_ctx *ctx, const char *fn, int64_t Q, int64_t N, int64_
     return AQ_OK;
 }
 
+// Room for an image that only a faster path reads, or null: an upload whose
+// device memory ends here is not refused, its calls take the per-stage
+// launches (AQ_EUCLID_TEST_NO_IMAGE, a test hook, ends it: at the image, or
+// behind it with the value "after").
+bool image_test_hook(bool after) {
+    const char *e = std::getenv("AQ_EUCLID_TEST_NO_IMAGE");
+    return e && (std::strcmp(e, "after") == 0) == after;
+}
+void *optional_image(size_t bytes) {
+    void *p = nullptr;
+    if (image_test_hook(false) || hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();   // not left for the next call to report
+        return nullptr;
+    }
+    return p;
+}
+
+// The codebook in fragment order, into d_cbx (enqueued).
+void euclid_fragment_image(aq_ctx *ctx, const aq_codebooks *cb) {
+    const int64_t pieces = cb->Q * cb->N * cb->K / 8;   // whole 16-code blocks: N is a multiple of the chunk
+    hipLaunchKernelGGL(euclid_fragments_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
+                       ctx->stream, reinterpret_cast<const u32x4 *>(cb->d_cbh), pieces, static_cast<int>(cb->K),
+                       reinterpret_cast<u32x4 *>(cb->d_cbx));
+}
+
 // A codebook set with its device buffers allocated, not yet filled.
-aq_status euclid_alloc(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, bool q8, bool any, int recipe,
+aq_status euclid_alloc(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, bool q8, bool any, bool image, int recipe,
                        aq_codebooks **out) {
     aq_codebooks *cb = new (std::nothrow) aq_codebooks();
     if (!cb) return aq_fail(ctx, AQ_E_NOMEM, "aq_euclid_upload: host allocation failed");
@@ -288,6 +313,7 @@ aq_status euclid_alloc(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, bool q8, bo
     bool ok = hipMalloc(&cb->d_cbh, QNK * 2) == hipSuccess && hipMalloc(&cb->d_cbl, QNK * 2) == hipSuccess &&
               hipMalloc(&cb->d_hh, QN * 4) == hipSuccess && hipMalloc(&cb->d_cbf, QNK * 4) == hipSuccess &&
               hipMalloc(&cb->d_bias, QN * 4) == hipSuccess && hipMalloc(&cb->d_e2, QN * 4) == hipSuccess;
+    if (ok && image) cb->d_cbx = static_cast<uint16_t *>(optional_image(QNK * 2));
     if (ok && q8) ok = hipMalloc(&cb->d_q8, QNK) == hipSuccess && hipMalloc(&cb->d_q8d, QNK / 32 * 4) == hipSuccess;
     if (!ok) {
         aq_euclid_release(cb);
@@ -356,6 +382,7 @@ aq_status euclid_prepare(aq_ctx *ctx, aq_codebooks *cb) {
         hipLaunchKernelGGL(euclid_prep_kernel, grid, block, 0, ctx->stream, cb->d_cbf, QN, cb->N,
                            static_cast<int>(cb->K), cb->d_cbh, cb->d_cbl, cb->d_hh, cb->d_bias, cb->d_e2, smax,
                            nonfinite);
+        if (cb->d_cbx) euclid_fragment_image(ctx, cb);
         step = "launch";
         e = hipGetLastError();
         if (e == hipSuccess) {
@@ -392,6 +419,10 @@ aq_status euclid_prepare(aq_ctx *ctx, aq_codebooks *cb) {
     int32_t nf;
     std::memcpy(&nf, &host[5 * cb->Q], 4);
     cb->exact_only = nf != 0;
+    if (cb->exact_only && cb->d_cbx) {   // every frame is scanned exactly: no call reads the image
+        (void)hipFree(cb->d_cbx);
+        cb->d_cbx = nullptr;
+    }
     // the per-stage bounds on the device, for the one-launch cascade
     std::vector<float> b3(static_cast<size_t>(3 * cb->Q));
     for (int64_t s = 0; s < cb->Q; ++s) {
@@ -406,34 +437,30 @@ aq_status euclid_prepare(aq_ctx *ctx, aq_codebooks *cb) {
     return st;
 }
 
-// Room for an image that only a faster path reads, or null: an upload whose
-// device memory ends here is not refused, its calls take the per-stage
-// launches (AQ_EUCLID_TEST_NO_IMAGE, a test hook, ends it).
-void *optional_image(size_t bytes) {
-    void *p = nullptr;
-    if (std::getenv("AQ_EUCLID_TEST_NO_IMAGE") || hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();   // not left for the next call to report
-        return nullptr;
+// A codebook set filled by `fill` and prepared.  plain: not the codebooks of
+// a projected set; the narrow cascade reads plain ones of K = 256 in fragment
+// order (allocated with the rest: on its own after the fill it took an upload
+// of 8 x 2 048 Q8_0 codes from 0.56 to 1.1 ms).  An upload that its memory
+// leaves without room is made again without it.
+template <typename Fill>
+aq_status euclid_build(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, bool q8, bool any, bool plain, int recipe, Fill fill,
+                       aq_codebooks **out) {
+    bool image = plain && !any && K == 256;
+    for (;;) {
+        aq_codebooks *cb = nullptr;
+        aq_status st = euclid_alloc(ctx, Q, N, K, q8, any, image, recipe, &cb);
+        if (st == AQ_OK && image && image_test_hook(true)) st = AQ_E_NOMEM;
+        if (st == AQ_OK) st = fill(cb);
+        if (st == AQ_OK) st = euclid_prepare(ctx, cb);
+        if (st == AQ_OK) {
+            *out = cb;
+            return AQ_OK;
+        }
+        if (cb) aq_euclid_release(cb);
+        if (st != AQ_E_NOMEM || !image) return st;
+        (void)hipGetLastError();
+        image = false;
     }
-    return p;
-}
-
-// The codebook in fragment order, for the one-launch cascades.
-aq_status euclid_fragment_image(aq_ctx *ctx, aq_codebooks *cb) {
-    const int64_t pieces = cb->Q * cb->N * cb->K / 8;   // whole 16-code blocks: N is a multiple of the chunk
-    cb->d_cbx = static_cast<uint16_t *>(optional_image(static_cast<size_t>(pieces) * 16));
-    if (!cb->d_cbx) return AQ_OK;
-    hipLaunchKernelGGL(euclid_fragments_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0,
-                       ctx->stream, reinterpret_cast<const u32x4 *>(cb->d_cbh), pieces, static_cast<int>(cb->K),
-                       reinterpret_cast<u32x4 *>(cb->d_cbx));
-    AQ_HIP(ctx, hipGetLastError());
-    AQ_HIP(ctx, hipStreamSynchronize(ctx->stream));   // the handle may be used on another stream
-    return AQ_OK;
-}
-// ... where the narrow cascade reads it: plain codebooks of K = 256 (a
-// codebook that is not finite is scanned exactly).
-aq_status euclid_narrow_image(aq_ctx *ctx, aq_codebooks *cb) {
-    return cb->K == 256 && !cb->any && !cb->exact_only ? euclid_fragment_image(ctx, cb) : AQ_OK;
 }
 
 aq_status euclid_upload_from(aq_ctx *ctx, const char *fn, int64_t Q, int64_t N, int64_t K, int cb_type,
@@ -444,17 +471,8 @@ aq_status euclid_upload_from(aq_ctx *ctx, const char *fn, int64_t Q, int64_t N, 
     aq_status st = check_upload(ctx, fn, Q, N, K, cb_type, recipe, &any);
     if (st != AQ_OK) return st;
     aq_device_guard g(ctx->device);
-    aq_codebooks *cb = nullptr;
-    st = euclid_alloc(ctx, Q, N, K, cb_type != AQ_CB_F32, any, recipe, &cb);
-    if (st == AQ_OK) st = euclid_fill(ctx, cb, cb_type, data, kind);
-    if (st == AQ_OK) st = euclid_prepare(ctx, cb);
-    if (st == AQ_OK && plain) st = euclid_narrow_image(ctx, cb);
-    if (st != AQ_OK) {
-        if (cb) aq_euclid_release(cb);
-        return st;
-    }
-    *out = cb;
-    return AQ_OK;
+    return euclid_build(ctx, Q, N, K, cb_type != AQ_CB_F32, any, plain, recipe,
+                        [&](aq_codebooks *cb) { return euclid_fill(ctx, cb, cb_type, data, kind); }, out);
 }
 
 }  // namespace
@@ -495,29 +513,24 @@ aq_status aq_euclid_upload_ema(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, con
     if (st != AQ_OK) return st;
     aq_device_guard g(ctx->device);
     const size_t QNK = static_cast<size_t>(Q * N * K), QN = static_cast<size_t>(Q * N);
-    aq_codebooks *cb = nullptr;
-    st = euclid_alloc(ctx, Q, N, K, false, any, recipe, &cb);
-    if (st != AQ_OK) return st;
     // the inputs go to the device once; the codebook is materialised straight
     // into the set's fp32 buffer and prepared there
-    float *d = nullptr;
-    if (hipMalloc(&d, (QNK + QN) * sizeof(float)) != hipSuccess) {
-        aq_euclid_release(cb);
-        return aq_fail(ctx, AQ_E_NOMEM, "aq_euclid_upload_ema: device allocation failed");
-    }
-    if (hipMemcpyAsync(d, embedding_sum, QNK * 4, hipMemcpyHostToDevice, ctx->stream) != hipSuccess ||
-        hipMemcpyAsync(d + QNK, cluster_usage, QN * 4, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
-        st = aq_fail(ctx, AQ_E_DEVICE, "aq_euclid_upload_ema: host to device copy failed");
-    if (st == AQ_OK) st = aq_ema_codebook(ctx, d, d + QNK, Q, N, K, eps, cb->d_cbf);
-    if (st == AQ_OK) st = euclid_prepare(ctx, cb);
-    if (st == AQ_OK) st = euclid_narrow_image(ctx, cb);
-    (void)hipFree(d);
-    if (st != AQ_OK) {
-        aq_euclid_release(cb);
-        return st;
-    }
-    *out = cb;
-    return AQ_OK;
+    auto fill = [&](aq_codebooks *cb) -> aq_status {
+        float *d = nullptr;
+        if (hipMalloc(&d, (QNK + QN) * sizeof(float)) != hipSuccess)
+            return aq_fail(ctx, AQ_E_NOMEM, "aq_euclid_upload_ema: device allocation failed");
+        aq_status fs = AQ_OK;
+        if (hipMemcpyAsync(d, embedding_sum, QNK * 4, hipMemcpyHostToDevice, ctx->stream) != hipSuccess ||
+            hipMemcpyAsync(d + QNK, cluster_usage, QN * 4, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
+            fs = aq_fail(ctx, AQ_E_DEVICE, "aq_euclid_upload_ema: host to device copy failed");
+        if (fs == AQ_OK) fs = aq_ema_codebook(ctx, d, d + QNK, Q, N, K, eps, cb->d_cbf);
+        const hipError_t e = hipStreamSynchronize(ctx->stream);
+        (void)hipFree(d);
+        if (fs == AQ_OK && e != hipSuccess)
+            fs = aq_fail(ctx, AQ_E_DEVICE, "aq_euclid_upload_ema: codebook kernel failed: %s", hipGetErrorString(e));
+        return fs;
+    };
+    return euclid_build(ctx, Q, N, K, false, any, true, recipe, fill, out);
 }
 
 aq_status aq_euclid_upload_projected(aq_ctx *ctx, int64_t Q, int64_t N, int64_t K, int64_t H, int cb_type,
@@ -554,8 +567,13 @@ aq_status aq_euclid_upload_projected(aq_ctx *ctx, int64_t Q, int64_t N, int64_t 
     // the one-launch cascade's images, for shapes that it takes
     if (st == AQ_OK && aq_proj_cascade_shape(cb->proj, N)) {
         cb->proj->w_cx = optional_image(aq_proj_cascade_bytes(cb->proj));
-        if (cb->proj->w_cx) st = aq_proj_cascade_weights(ctx, cb->proj);
-        if (st == AQ_OK && cb->proj->w_cx) st = euclid_fragment_image(ctx, cb);
+        if (cb->proj->w_cx) cb->d_cbx = static_cast<uint16_t *>(optional_image(static_cast<size_t>(Q * N * K) * 2));
+        if (cb->d_cbx) {
+            st = aq_proj_cascade_weights(ctx, cb->proj);
+            euclid_fragment_image(ctx, cb);
+            if (st == AQ_OK && (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess))
+                st = aq_fail(ctx, AQ_E_DEVICE, "aq_euclid_upload_projected: codebook image failed");
+        }
     }
     if (st != AQ_OK) {
         aq_euclid_release(cb);

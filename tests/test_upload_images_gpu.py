@@ -1,6 +1,7 @@
 """The images that an upload builds for the one-launch cascades alone: an
-upload without memory for them is not refused and its calls give the same
-bits through the per-stage launches (AQ_EUCLID_TEST_NO_IMAGE ends the memory),
+upload without memory for them, or for what comes after them, is not refused
+and its calls give the same bits through the per-stage launches
+(AQ_EUCLID_TEST_NO_IMAGE ends the memory),
 and shapes that those cascades do not take hold none."""
 
 import numpy as np
@@ -29,17 +30,22 @@ def encode(torch, cbs, x, want_launches):
     return idx.cpu().numpy(), res.cpu().numpy().view(np.uint32)
 
 
-@pytest.mark.parametrize("kind", ["plain", "ema", "projected", "projected_q8"])
-def test_upload_without_memory_for_images(torch, monkeypatch, kind):
+@pytest.mark.parametrize("kind,ends", [
+    ("plain", "at"), ("plain", "after"), ("q8", "at"), ("ema", "at"), ("ema", "after"), ("projected", "at"),
+    ("projected_q8", "at")])
+def test_upload_without_memory_for_images(torch, monkeypatch, kind, ends):
     import aqmi
     from aqmi import synth
 
-    print(f"[gpu] upload images {kind}", flush=True)
+    print(f"[gpu] upload images {kind} {ends}", flush=True)
     ctx, Q, M = aqmi.Context(0), 3, 70
 
     def upload():
         if kind == "plain":
             return aqmi.Codebooks(ctx, synth.normal(95, 1, (Q, 256, 256)), aqmi.OMNIVOICE)
+        if kind == "q8":
+            blocks = np.stack([synth.q8_0_random_codebook(95, 10 + s, 256, 256) for s in range(Q)])
+            return aqmi.Codebooks(ctx, blocks, aqmi.HIGGS, aqmi.CB_Q8_0)
         if kind == "ema":
             return aqmi.Codebooks.from_ema(ctx, synth.normal(95, 1, (Q, 256, 256)), np.ones((Q, 256), np.float32),
                                            aqmi.DIRECT)
@@ -52,7 +58,7 @@ def test_upload_without_memory_for_images(torch, monkeypatch, kind):
     cbs = upload()
     x = torch.from_numpy(synth.normal(95, 2, (M, cbs.H))).cuda()
     want = encode(torch, cbs, x, 1)
-    monkeypatch.setenv("AQ_EUCLID_TEST_NO_IMAGE", "1")
+    monkeypatch.setenv("AQ_EUCLID_TEST_NO_IMAGE", ends)
     got = encode(torch, upload(), x, Q)
     assert np.array_equal(got[0], want[0])
     assert np.array_equal(got[1], want[1])

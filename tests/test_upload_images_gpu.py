@@ -82,6 +82,8 @@ def test_no_image_where_no_call_reads_it(torch):
     # three values per code
     need = Q * (N * K * 8 + N * H * 4 + 2 * K * H * 4 + N * 12)
     print(f"held {held}, needed {need}", flush=True)
-    assert need <= held + (2 << 20)
+    # the three 1 MiB buffers of values per code can lie in a chunk that the
+    # process holds already; the others are 16 MiB at least
+    assert held >= need - 3 * Q * N * 4 - (2 << 20)
     assert held < need + (32 << 20)   # the allocator's rounding of ten buffers
     del one, cbs

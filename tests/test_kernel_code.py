@@ -20,7 +20,7 @@ OBJDUMP = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
 
 # Kernels that must hold no loop through the execution mask where they spill,
 # and the most vector registers that each may spill.
-SPILLS = {"euclid_refine_select_kernel": 0, "euclid_narrow_kernel": 36, "proj_cascade_kernel": 78,
+SPILLS = {"euclid_refine_select_kernel": 0, "euclid_narrow_kernel": 28, "proj_cascade_kernel": 78,
           "euclid_cascade_kernel": 67}
 
 

@@ -3504,22 +3504,16 @@ __global__ __launch_bounds__(kNwThreads, 1) void euclid_narrow_kernel(CascadeArg
     const int nblk = N / 16;
     const int nb = wave < nblk ? (nblk - wave + kNwWaves - 1) / kNwWaves : 0;   // this wave's 16-code blocks
 
-    // The stage-0 input (rows past M read row M - 1).  Up to two frame groups
-    // every load of a thread is on its way before the first is stored (6 800
-    // Q8_0 frames of four stages 71.2 us one by one, 67.6 so; a 197-frame clip of 16
-    // stages 264.8, 263.3); of four groups one by one (48 000 frames 512 us, 514
-    // with four at once).
-    auto row_in = [&](int e0) {
+    // The stage-0 input (rows past M read row M - 1), four loads of a thread on
+    // their way before the first is stored (one by one / so: 6 800 Q8_0 frames
+    // of 4 stages 71.2 / 67.6 us, a 197-frame clip of 16 stages 264.8 / 263.3;
+    // 48 000 frames of 8 stages, Higgs 479 / 465, DIRECT 512 / 507, OmniVoice 497 /
+    // 495, Q8_0 508 / 510).
+#pragma unroll 4
+    for (int e0 = 0; e0 < LY::FRAMES * (K / 4); e0 += kNwThreads) {
         const int e = e0 + threadIdx.x, f = e / (K / 4), k = e % (K / 4) * 4;
         const int64_t m = m_tile + f < M ? m_tile + f : M - 1;
         *reinterpret_cast<f32x4 *>(xr + f * LY::XSTR + k) = *reinterpret_cast<const f32x4 *>(c.x0 + m * K + k);
-    };
-    if constexpr (FG < 4) {
-#pragma unroll
-        for (int e0 = 0; e0 < LY::FRAMES * (K / 4); e0 += kNwThreads) row_in(e0);
-    } else {
-#pragma unroll 1
-        for (int e0 = 0; e0 < LY::FRAMES * (K / 4); e0 += kNwThreads) row_in(e0);
     }
 
     typename MX::V8 ring[R];

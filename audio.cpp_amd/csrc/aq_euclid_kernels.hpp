@@ -3459,6 +3459,53 @@ struct NwLayout {
     static_assert(BYTES <= static_cast<int>(kAqLdsBytes), "a block's LDS");
 };
 
+// What the certificate rests on, shared with the projected cascade's search.
+//
+// Eight elements of the lane's frame as fp16, with the K-slice's part of the
+// rounding norms: sx = |x~|^2, sd = |x - x~|^2, sxx = |x|^2 over the frame's
+// four lanes.
+__device__ __forceinline__ u32x4 pack_slice(const float (&v)[8], float &sx, float &sd, float &sxx) {
+    using MX = Mx;
+    u32x4 packed;
+    sx = sd = sxx = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const float v0 = v[2 * t], v1 = v[2 * t + 1];
+        const typename MX::V2 pr = {static_cast<typename MX::E>(v0), static_cast<typename MX::E>(v1)};
+        const unsigned w = __builtin_bit_cast(unsigned, pr);
+        packed[t] = w;
+        const float r0 = MX::lo(w), r1 = MX::hi(w);
+        sx = __fmaf_rn(r0, r0, sx);
+        sx = __fmaf_rn(r1, r1, sx);
+        const float d0 = v0 - r0, d1 = v1 - r1;
+        sd = __fmaf_rn(d0, d0, sd);
+        sd = __fmaf_rn(d1, d1, sd);
+        sxx = __fmaf_rn(v0, v0, sxx);
+        sxx = __fmaf_rn(v1, v1, sxx);
+    }
+    sx = rows_sum(sx);
+    sd = rows_sum(sd);
+    sxx = rows_sum(sxx);
+    return packed;
+}
+
+// A key into a lane's sorted list, whose last key bounds what it drops.
+template <int TS>
+__device__ __forceinline__ void insert_key(float key, float (&top)[TS]) {
+#pragma unroll
+    for (int j = TS - 1; j > 0; --j) top[j] = __builtin_amdgcn_fmed3f(top[j - 1], top[j], key);
+    top[0] = __builtin_amdgcn_fmed3f(top[0], key, 3.40282347e38f);
+}
+
+// One key of a wave's list into the merged list mt; taul grows to a bound on
+// every key that the wave (last: its list's last key) or the merge dropped.
+template <int TOPL>
+__device__ __forceinline__ void merge_key(float key, bool last, float (&mt)[TOPL], float &taul) {
+    if (last) taul = fmaxf(taul, key);
+    taul = fmaxf(taul, fminf(mt[TOPL - 1], key));
+    insert_key(key, mt);
+}
+
 template <int RECIPE, bool Q8, int KS, int FG, int TOPL>
 __global__ __launch_bounds__(kNwThreads, 1) void euclid_narrow_kernel(CascadeArgs c) {
     using T = Tile<KS>;
@@ -3562,27 +3609,8 @@ __global__ __launch_bounds__(kNwThreads, 1) void euclid_narrow_kernel(CascadeArg
                     const int f = g * 16 + col;
                     q8_image_block(v, xq + f * LY::XQS + ks * 32 + kq * 8, xd + f * KS + ks);
                 }
-                u32x4 packed;
-                float sx = 0.0f, sd = 0.0f, sxx = 0.0f;
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const float v0 = v[2 * t], v1 = v[2 * t + 1];
-                    const typename MX::V2 pr = {static_cast<typename MX::E>(v0), static_cast<typename MX::E>(v1)};
-                    const unsigned w = __builtin_bit_cast(unsigned, pr);
-                    packed[t] = w;
-                    const float r0 = MX::lo(w), r1 = MX::hi(w);
-                    sx = __fmaf_rn(r0, r0, sx);
-                    sx = __fmaf_rn(r1, r1, sx);
-                    const float d0 = v0 - r0, d1 = v1 - r1;
-                    sd = __fmaf_rn(d0, d0, sd);
-                    sd = __fmaf_rn(d1, d1, sd);
-                    sxx = __fmaf_rn(v0, v0, sxx);
-                    sxx = __fmaf_rn(v1, v1, sxx);
-                }
-                xh[(g * KS + ks) * kWave + lane] = packed;
-                sx = rows_sum(sx);
-                sd = rows_sum(sd);
-                sxx = rows_sum(sxx);
+                float sx, sd, sxx;
+                xh[(g * KS + ks) * kWave + lane] = pack_slice(v, sx, sd, sxx);
                 if (kq == 0) {
                     float *n3 = nrm + ks * 3 * LY::FRAMES + g * 16 + col;
                     n3[0] = sx;
@@ -3617,12 +3645,7 @@ __global__ __launch_bounds__(kNwThreads, 1) void euclid_narrow_kernel(CascadeArg
                 unsigned local = local0 + i;
                 asm("" : "+s"(local));
 #pragma unroll
-                for (int g = 0; g < FG; ++g) {
-                    const float key = key_of(acc[g][i], local, vkeep);
-#pragma unroll
-                    for (int j = TS - 1; j > 0; --j) top[g][j] = __builtin_amdgcn_fmed3f(top[g][j - 1], top[g][j], key);
-                    top[g][0] = __builtin_amdgcn_fmed3f(top[g][0], key, 3.40282347e38f);
-                }
+                for (int g = 0; g < FG; ++g) insert_key(key_of(acc[g][i], local, vkeep), top[g]);
             }
         };
         for (int i0 = 0; i0 < nb; i0 += U) {
@@ -3658,15 +3681,7 @@ __global__ __launch_bounds__(kNwThreads, 1) void euclid_narrow_kernel(CascadeArg
 #pragma unroll
         for (int w = 0; w < kNwWaves; ++w)
 #pragma unroll
-            for (int j = 0; j < TS; ++j) {
-                const float key = keys[((w * FG + g) * TS + j) * kWave + lane];
-                if (j == TS - 1) taul = fmaxf(taul, key);
-                // what the merged list drops bounds the rest too
-                taul = fmaxf(taul, fminf(mt[TOPL - 1], key));
-#pragma unroll
-                for (int i = TOPL - 1; i > 0; --i) mt[i] = __builtin_amdgcn_fmed3f(mt[i - 1], mt[i], key);
-                mt[0] = __builtin_amdgcn_fmed3f(mt[0], key, 3.40282347e38f);
-            }
+            for (int j = 0; j < TS; ++j) merge_key(keys[((w * FG + g) * TS + j) * kWave + lane], j == TS - 1, mt, taul);
         float n3[3];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {

@@ -405,42 +405,23 @@ __device__ __attribute__((noinline)) void scan_open(const float *cbf, const floa
     __syncthreads();
 }
 
-// The search's parts below are the narrow cascade's (euclid_narrow_kernel) for
-// one group of frames; as shared code they cost its widest tile 10 to 25
-// spilled registers and 13 % at 6 000 frames, so that it keeps its own.
+// The search's loops are the narrow cascade's (euclid_narrow_kernel) for one
+// group of frames: as shared code they cost its widest tile 10 to 25 spilled
+// registers and 13 % at 6 000 frames, so that it keeps its own.  What the
+// certificate rests on is shared: pack_slice, insert_key, merge_key.
 //
 // K-slice ks of 16 frames' fp32 rows (xrow: the lane's frame's row) as fp16
 // fragments, with the slice's part of the rounding norms |x~|^2, |x - x~|^2,
 // |x|^2 (n3[0], n3[stride], n3[2 stride], written for the lane's frame by its
-// first lane).  A Q8_0 codebook scores the query's Q8_0 image; its quants
-// and scale go to xq and xd where given.
+// first lane).  A Q8_0 codebook scores the query's Q8_0 image.
 template <bool Q8>
-__device__ inline u32x4 fragment_slice(const float *xrow, int ks, int kq, float *n3, int stride, int8_t *xq, float *xd) {
-    using MX = Mx;
+__device__ inline u32x4 fragment_slice(const float *xrow, int ks, int kq, float *n3, int stride) {
     const float *row = xrow + ks * 32 + kq * 8;
     const f32x4 lo = *reinterpret_cast<const f32x4 *>(row), hi = *reinterpret_cast<const f32x4 *>(row + 4);
     float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    if (Q8) q8_image_block(v, xq, xd);
-    u32x4 packed;
-    float sx = 0.0f, sd = 0.0f, sxx = 0.0f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const float v0 = v[2 * t], v1 = v[2 * t + 1];
-        const typename MX::V2 pr = {static_cast<typename MX::E>(v0), static_cast<typename MX::E>(v1)};
-        const unsigned w = __builtin_bit_cast(unsigned, pr);
-        packed[t] = w;
-        const float r0 = MX::lo(w), r1 = MX::hi(w);
-        sx = __fmaf_rn(r0, r0, sx);
-        sx = __fmaf_rn(r1, r1, sx);
-        const float d0 = v0 - r0, d1 = v1 - r1;
-        sd = __fmaf_rn(d0, d0, sd);
-        sd = __fmaf_rn(d1, d1, sd);
-        sxx = __fmaf_rn(v0, v0, sxx);
-        sxx = __fmaf_rn(v1, v1, sxx);
-    }
-    sx = rows_sum(sx);
-    sd = rows_sum(sd);
-    sxx = rows_sum(sxx);
+    if (Q8) q8_image_block(v);
+    float sx, sd, sxx;
+    const u32x4 packed = pack_slice(v, sx, sd, sxx);
     if (kq == 0) {
         n3[0] = sx;
         n3[stride] = sd;
@@ -450,8 +431,8 @@ __device__ inline u32x4 fragment_slice(const float *xrow, int ks, int kq, float 
 }
 
 // One wave's share of a codebook in fragment order: the 16-code blocks wave,
-// wave + NW, ..., contracted with FG groups of fragments, R fragments ahead.
-template <int KS, int FG, int TS, int R, int NW>
+// wave + NW, ..., contracted with the frames' fragments, R fragments ahead.
+template <int KS, int TS, int R, int NW>
 struct CodeStream {
     using MX = Mx;
     static constexpr int U = R > KS ? R / KS : 1;   // 16-code blocks per unrolled step
@@ -487,24 +468,18 @@ struct CodeStream {
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    __device__ void sweep(const uint16_t *cbx, const float *nhh, const typename MX::V8 (&xb)[FG][KS], float (&top)[FG][TS],
-                          unsigned vkeep) {
+    __device__ void sweep(const uint16_t *cbx, const float *nhh, const typename MX::V8 (&xb)[KS], float (&top)[TS], unsigned vkeep) {
 #pragma unroll
-        for (int g = 0; g < FG; ++g)
-#pragma unroll
-            for (int j = 0; j < TS; ++j) top[g][j] = -INFINITY;
+        for (int j = 0; j < TS; ++j) top[j] = -INFINITY;
         for (int i0 = 0; i0 < nb; i0 += U) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                f32x4 acc[FG];
-#pragma unroll
-                for (int g = 0; g < FG; ++g) acc[g] = hring[u];
+                f32x4 acc = hring[u];
                 hring[u] = load_h(nhh, i0 + u + U);
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
                     const int p = u * KS + ks;
-#pragma unroll
-                    for (int g = 0; g < FG; ++g) acc[g] = MX::mfma(ring[p % R], xb[g][ks], acc[g]);
+                    acc = MX::mfma(ring[p % R], xb[ks], acc);
                     ring[p % R] = load_a(cbx, i0 + (p + R) / KS, (p + R) % KS);
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -516,39 +491,12 @@ struct CodeStream {
                     // v_and_or_b32
                     unsigned local = local0 + i;
                     asm("" : "+s"(local));
-#pragma unroll
-                    for (int g = 0; g < FG; ++g) {
-                        const float key = key_of(acc[g][i], local, vkeep);
-#pragma unroll
-                        for (int j = TS - 1; j > 0; --j) top[g][j] = __builtin_amdgcn_fmed3f(top[g][j - 1], top[g][j], key);
-                        top[g][0] = __builtin_amdgcn_fmed3f(top[g][0], key, 3.40282347e38f);
-                    }
+                    insert_key(key_of(acc[i], local, vkeep), top);
                 }
             }
         }
     }
 };
-
-// The lane's key lists of NW waves (keys[w][FG][TS][64], group g) merged into
-// mt; returns a bound on every key that a wave or the merge dropped.
-template <int NW, int FG, int TS, int TOPL>
-__device__ inline float merge_keys(const float *keys, int g, int lane, float (&mt)[TOPL]) {
-    float taul = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < TOPL; ++j) mt[j] = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < NW; ++w)
-#pragma unroll
-        for (int j = 0; j < TS; ++j) {
-            const float key = keys[((w * FG + g) * TS + j) * kWave + lane];
-            if (j == TS - 1) taul = fmaxf(taul, key);
-            taul = fmaxf(taul, fminf(mt[TOPL - 1], key));
-#pragma unroll
-            for (int i = TOPL - 1; i > 0; --i) mt[i] = __builtin_amdgcn_fmed3f(mt[i - 1], mt[i], key);
-            mt[0] = __builtin_amdgcn_fmed3f(mt[0], key, 3.40282347e38f);
-        }
-    return taul;
-}
 
 template <int RECIPE, bool Q8C, bool Q8W, int F, int TOPL>
 __global__ __launch_bounds__(kPcThreads, 2) void proj_cascade_kernel(PcArgs pa) {
@@ -656,23 +604,28 @@ __global__ __launch_bounds__(kPcThreads, 2) void proj_cascade_kernel(PcArgs pa) 
         } else {
             project_f32<F>(pa.wx + static_cast<int64_t>(s) * kPcK * H, bias, lrows, H, (lds_float *)p);
         }
-        CodeStream<kPcKS, 1, TOPL, R, kPcWaves> codes(N, wave, lane);
+        CodeStream<kPcKS, TOPL, R, kPcWaves> codes(N, wave, lane);
         codes.fill(cbx, a.nhh);
         __syncthreads();
         // ---- search ----
         if (wave < kPcKS)
-            xh[wave * kWave + lane] = fragment_slice<Q8C>(p + col * XSTR, wave, kq, nrm + wave * 3 * 16 + col, 16, nullptr, nullptr);
+            xh[wave * kWave + lane] = fragment_slice<Q8C>(p + col * XSTR, wave, kq, nrm + wave * 3 * 16 + col, 16);
         __syncthreads();
-        typename Mx::V8 xb[1][kPcKS];
+        typename Mx::V8 xb[kPcKS];
 #pragma unroll
-        for (int ks = 0; ks < kPcKS; ++ks) xb[0][ks] = __builtin_bit_cast(typename Mx::V8, xh[ks * kWave + lane]);
-        float top[1][TOPL];
+        for (int ks = 0; ks < kPcKS; ++ks) xb[ks] = __builtin_bit_cast(typename Mx::V8, xh[ks * kWave + lane]);
+        float top[TOPL];
         codes.sweep(cbx, a.nhh, xb, top, vkeep);
 #pragma unroll
-        for (int j = 0; j < TOPL; ++j) keys[(wave * TOPL + j) * kWave + lane] = top[0][j];
+        for (int j = 0; j < TOPL; ++j) keys[(wave * TOPL + j) * kWave + lane] = top[j];
         __syncthreads();
-        float mt[TOPL], n3[3];
-        const float taul = merge_keys<kPcWaves, 1, TOPL, TOPL>(keys, 0, lane, mt);
+        float mt[TOPL], taul = -INFINITY, n3[3];
+#pragma unroll
+        for (int j = 0; j < TOPL; ++j) mt[j] = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < kPcWaves; ++w)
+#pragma unroll
+            for (int j = 0; j < TOPL; ++j) merge_key(keys[(w * TOPL + j) * kWave + lane], j == TOPL - 1, mt, taul);
 #pragma unroll
         for (int q = 0; q < 3; ++q) n3[q] = nrm[q * 16 + col] + nrm[(3 + q) * 16 + col];
         __syncthreads();   // keys and fragments are read: the select queues take their place

@@ -468,7 +468,8 @@ struct CodeStream {
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    __device__ void sweep(const uint16_t *cbx, const float *nhh, const typename MX::V8 (&xb)[KS], float (&top)[TS], unsigned vkeep) {
+    __device__ void sweep(const uint16_t *cbx, const float *nhh, const typename MX::V8 (&xb)[KS], float (&top)[TS],
+                          unsigned vkeep) {
 #pragma unroll
         for (int j = 0; j < TS; ++j) top[j] = -INFINITY;
         for (int i0 = 0; i0 < nb; i0 += U) {
